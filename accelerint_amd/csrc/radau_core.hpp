@@ -388,43 +388,84 @@ __device__ __forceinline__ void group_argmax(T& bv, int& bkey) {
 }
 
 
-// FP32 pivot search of the register LU at G = 64: (value, key) packed in one
-// 64-bit integer -- high word the bits of the value (non-negative floats
-// order as unsigned integers), low word ~key (a smaller key gives a larger
-// word); candidates that are inactive or NaN get 0 : ~0x7fffffff, below every
-// active one, as in group_argmax's order, where they never win.  Keys are
-// unique, so the maximum is the same winner group_argmax finds, with one
-// 64-bit compare per exchange.  Returns the winner's key (0x7fffffff: none).
+// Pivot search of the register LU at G = 64, one row per lane (row = lane):
+// the first maximum of the magnitudes v over the active lanes in LAPACK's row
+// order (pos), as a wave-uniform lane, or -1 if no active lane holds a
+// comparable value (every candidate NaN).  The magnitudes are compared as
+// integers (non-negative floats order as their bits); only the leading 32 bits
+// go through the lane exchanges, one v_max_u32 per exchange, and the lanes that
+// attain the maximum come out of one compare as a scalar mask.  Lanes that agree
+// in those bits, which is rare, are compared one by one in full.  Against an
+// exchange of (value, key) pairs joined through scalar mask logic this is ~20
+// instead of 84 instructions per FP64 search.
+__device__ __forceinline__ unsigned mag_hi(float v) { return __float_as_uint(v); }
+__device__ __forceinline__ unsigned mag_hi(double v) { return (unsigned)__double2hiint(v); }
+__device__ __forceinline__ unsigned max_u(unsigned a, unsigned b) { return a > b ? a : b; }
 template <int CTRL>
-__device__ __forceinline__ unsigned long long dpp_u64(unsigned long long v) {
-  const unsigned lo = (unsigned)dpp_i<CTRL>((int)(unsigned)v);
-  const unsigned hi = (unsigned)dpp_i<CTRL>((int)(unsigned)(v >> 32));
-  return ((unsigned long long)hi << 32) | lo;
+__device__ __forceinline__ unsigned dpp_max_u(unsigned v) {
+  return max_u(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, false));
 }
-__device__ __forceinline__ int pivot_key64(float v, int key, bool act) {
-  unsigned long long p = (act && v == v) ? (((unsigned long long)__float_as_uint(v) << 32) | (unsigned)~key)
-                                         : (unsigned long long)(unsigned)~0x7fffffff;
-  const auto mx = [](unsigned long long a, unsigned long long b) { return a > b ? a : b; };
-  p = mx(p, dpp_u64<kDppXor1>(p));
-  p = mx(p, dpp_u64<kDppXor2>(p));
-  p = mx(p, dpp_u64<kDppHalfMirror>(p));
-  p = mx(p, dpp_u64<kDppMirror>(p));
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    int lo0 = (int)(unsigned)p, lo1 = lo0, hi0 = (int)(unsigned)(p >> 32), hi1 = hi0;
-    if (h == 0) {
-      swap_row_pairs(lo0, lo1);
-      swap_row_pairs(hi0, hi1);
-    } else {
-      swap_halves(lo0, lo1);
-      swap_halves(hi0, hi1);
+template <class T>
+__device__ __forceinline__ int wave_pivot(T v, int pos, bool act) {
+  const unsigned key = act && v == v ? mag_hi(v) + 1u : 0u;  // 0: no candidate
+  unsigned m = dpp_max_u<kDppXor1>(key);
+  m = dpp_max_u<kDppXor2>(m);
+  m = dpp_max_u<kDppHalfMirror>(m);
+  m = dpp_max_u<kDppMirror>(m);
+  int x = (int)m, y = (int)m;
+  swap_row_pairs(x, y);
+  x = y = (int)max_u((unsigned)x, (unsigned)y);
+  swap_halves(x, y);
+  m = (unsigned)__builtin_amdgcn_readfirstlane((int)max_u((unsigned)x, (unsigned)y));
+  unsigned long long cand = __builtin_amdgcn_ballot_w64(key == m);
+  int lane = (int)__builtin_ctzll(cand);  // (the lane that holds the maximum: never empty)
+  if (__builtin_expect((cand & (cand - 1)) != 0, 0)) {
+    if (m == 0) return -1;
+    lane = -1;
+    T bv = T(0);
+    int best = 0;
+    while (cand) {
+      const int l = (int)__builtin_ctzll(cand);
+      cand &= cand - 1;
+      const T w = Grp<64>::bcast(v, l);
+      const int q = __builtin_amdgcn_readlane(pos, l);
+      if (lane < 0 || w > bv || (w == bv && q < best)) {
+        bv = w;
+        best = q;
+        lane = l;
+      }
     }
-    const unsigned long long a = ((unsigned long long)(unsigned)hi0 << 32) | (unsigned)lo0;
-    const unsigned long long b = ((unsigned long long)(unsigned)hi1 << 32) | (unsigned)lo1;
-    p = mx(a, b);
+    lane = __builtin_amdgcn_readfirstlane(lane);
   }
-  return (int)~(unsigned)p;
+  return lane;
 }
+
+// Tests of a wave-uniform pivot on its bits, in scalar registers.
+__device__ __forceinline__ bool is_zero(float v) { return (__float_as_uint(v) & 0x7fffffffu) == 0; }
+__device__ __forceinline__ bool is_zero(double v) {
+  return (((unsigned)__double2hiint(v) & 0x7fffffffu) | (unsigned)__double2loint(v)) == 0;
+}
+__device__ __forceinline__ bool is_subnormal_or_zero(double v) {
+  return ((unsigned)__double2hiint(v) & 0x7fffffffu) < 0x00100000u;
+}
+
+// Keeps a value where it is computed: the compiler neither moves its
+// computation past this point nor recomputes or specializes it later (v: a
+// vector register, s: a scalar one, for wave-uniform values).
+template <class T>
+__device__ __forceinline__ void pin(T& v) {
+  __asm__ volatile("" : "+v"(v));
+}
+template <class T>
+__device__ __forceinline__ void pin_s(T& v) {
+  v = (T)__builtin_amdgcn_readfirstlane((int)v);
+  __asm__ volatile("" : "+s"(v));
+}
+// Columns whose pivot-row entries are in scalar registers at once (the
+// schedule of a step is cut after every such chunk): more of them at once
+// overflow the 102 scalar registers, and every spilled broadcast costs two
+// lane moves.
+constexpr int kBcastChunk = 8;
 
 // Group all-reduce of a sum.  16- and 64-lane groups: DPP pairs within rows
 // (each pair adds the same two operands, so the lanes of a row agree bit for
@@ -466,27 +507,81 @@ __device__ __forceinline__ void lu_init(int (&pos)[R], T (&rd)[R], int& info) {
   info = 0;
 }
 
-// Elimination step k of the real LU (k a compile-time constant after unrolling).
+// Elimination step k of the real LU, a wavefront per matrix and a row per lane
+// (k a compile-time constant after unrolling): the operations of lu_real_step
+// below in the same order.  Bound by the issue of a lane move per broadcast
+// pivot-row word and the step's chain search -> reciprocal -> multiplier.  What
+// a step leaves behind (multipliers, reciprocal, positions, pivot row) is
+// pinned to the step and the trailing update is cut into chunks of columns:
+// left alone, the compiler delayed the selects and updates of each step past
+// the next one's branches, which kept up to 54 broadcasts alive in scalar
+// registers (spilled by two lane moves each) and gave every step scratch slots.
+// With the solves' SolveView, order 54, 32768 conditions of one global step:
+// FP64 265 -> 117 ms (scratch 2816 -> 784 B a lane, lane moves 17000 -> 11700),
+// FP32 factors on 65536 conditions 253 -> 186 ms (scratch 912 -> 0 B).
+template <int N, class T>
+__device__ __forceinline__ void wave_lu_real_step(const int k, T (&a)[N], int& pos, Perm<N>& perm, T& rd, int& info) {
+  const int ln = Grp<64>::lane();
+  const int win = wave_pivot(fabs(a[k]), pos, pos >= k);
+  const int plane = win & 63;
+  const int prow = win >= 0 ? win : 0xff;
+  const int pp = __builtin_amdgcn_readlane(pos, plane);
+  const int ppos = win >= 0 ? pp : 0x7fffff;
+  perm.set(k, prow);
+  pin_s(perm.w[k >> 2]);
+  const T piv = Grp<64>::bcast(a[k], plane);
+  const bool nz = !is_zero(piv);
+  info = !nz && info == 0 ? k + 1 : info;
+  pin(info);
+  const bool is_piv = ln == prow;
+  pos = is_piv ? k : (pos == k ? ppos : pos);  // LAPACK swaps rows k and ppos
+  pin(pos);
+  const T rp = recip(piv);
+  T lq = a[k] * rp;
+  // LAPACK divides instead of scaling by the reciprocal when |pivot| < sfmin
+  // (FP64 path only; the FP32 factors need no such care)
+  if constexpr (std::is_same<T, double>::value)
+    if (__builtin_expect(is_subnormal_or_zero(piv), 0)) lq = a[k] / piv;
+  rd = is_piv ? (nz ? rp : T(0)) : rd;
+  pin(rd);
+  const bool act = nz && pos > k;
+  a[k] = act ? lq : a[k];
+  T l = act ? -lq : T(-0.0);
+  pin(a[k]);
+  pin(l);
+#pragma unroll
+  for (int j0 = k + 1; j0 < N; j0 += kBcastChunk) {
+    __builtin_amdgcn_sched_barrier(0);
+    T u[kBcastChunk];
+#pragma unroll
+    for (int j = j0; j < j0 + kBcastChunk; ++j)
+      if (j < N) u[j - j0] = Grp<64>::bcast(a[j], plane);
+#pragma unroll
+    for (int j = j0; j < j0 + kBcastChunk; ++j)
+      if (j < N) {
+        a[j] = fma(l, u[j - j0], a[j]);
+        pin(a[j]);
+      }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+}
+
 template <int N, int G, int R, class T>
 __device__ __forceinline__ void lu_real_step(const int k, T (&a)[R][N], int (&pos)[R], Perm<N>& perm,
                                              T (&rd)[R], int& info) {
   const int ln = Grp<G>::lane();
   int bkey = 0x7fffffff;
-  if constexpr (G == 64 && R == 1 && std::is_same<T, float>::value) {
-    bkey = pivot_key64(fabs(a[0][k]), (pos[0] << 8) | Rows<N, G, R>::row(ln, 0), pos[0] >= k);
-  } else {
-    T bv = T(-1);
+  T bv = T(-1);
 #pragma unroll
-    for (int q = 0; q < R; ++q) {
-      const bool act = pos[q] >= k;
-      const T v = fabs(a[q][k]);
-      const int key = (pos[q] << 8) | Rows<N, G, R>::row(ln, q);
-      const bool better = act && (v > bv || (v == bv && key < bkey));
-      bv = better ? v : bv;
-      bkey = better ? key : bkey;
-    }
-    group_argmax<G>(bv, bkey);
+  for (int q = 0; q < R; ++q) {
+    const bool act = pos[q] >= k;
+    const T v = fabs(a[q][k]);
+    const int key = (pos[q] << 8) | Rows<N, G, R>::row(ln, q);
+    const bool better = act && (v > bv || (v == bv && key < bkey));
+    bv = better ? v : bv;
+    bkey = better ? key : bkey;
   }
+  group_argmax<G>(bv, bkey);
   const int prow = bkey & 0xff;
   const int ppos = bkey >> 8;
   const int plane = prow % G;
@@ -533,31 +628,95 @@ template <int N, int G, int R, class T>
 __device__ __forceinline__ void lu_real(T (&a)[R][N], int (&pos)[R], Perm<N>& perm,
                                         T (&rd)[R], int& info) {
   lu_init<N, G, R, T>(pos, rd, info);
+  if constexpr (G == 64 && R == 1) {
+    Perm<N> pm = {};  // built in scalar registers
+    int inf = 0;
 #pragma unroll
-  for (int k = 0; k < N; ++k) lu_real_step<N, G, R, T>(k, a, pos, perm, rd, info);
+    for (int k = 0; k < N; ++k) wave_lu_real_step<N, T>(k, a[0], pos[0], pm, rd[0], inf);
+    perm = pm;
+    info = inf;
+  } else {
+#pragma unroll
+    for (int k = 0; k < N; ++k) lu_real_step<N, G, R, T>(k, a, pos, perm, rd, info);
+  }
 }
 
 // ---- complex LU (zgetf2 semantics) -------------------------------------------
+// (a wavefront per matrix, a row per lane: as wave_lu_real_step)
+template <int N, class T>
+__device__ __forceinline__ void wave_lu_cplx_step(const int k, T (&ar)[N], T (&ai)[N], int& pos, Perm<N>& perm, T& rdr,
+                                                  T& rdi, int& info) {
+  const int ln = Grp<64>::lane();
+  const int win = wave_pivot(fabs(ar[k]) + fabs(ai[k]), pos, pos >= k);
+  const int plane = win & 63;
+  const int prow = win >= 0 ? win : 0xff;
+  const int pp = __builtin_amdgcn_readlane(pos, plane);
+  const int ppos = win >= 0 ? pp : 0x7fffff;
+  perm.set(k, prow);
+  pin_s(perm.w[k >> 2]);
+  const T pr_ = Grp<64>::bcast(ar[k], plane);
+  const T pi_ = Grp<64>::bcast(ai[k], plane);
+  const bool nz = !(is_zero(pr_) && is_zero(pi_));
+  info = !nz && info == 0 ? k + 1 : info;
+  pin(info);
+  const bool is_piv = ln == prow;
+  pos = is_piv ? k : (pos == k ? ppos : pos);
+  pin(pos);
+  T rr, ri;
+  crecip(pr_, pi_, rr, ri);
+  rdr = is_piv ? (nz ? rr : T(0)) : rdr;
+  rdi = is_piv ? (nz ? ri : T(0)) : rdi;
+  pin(rdr);
+  pin(rdi);
+  const bool act = nz && pos > k;
+  const T xr = ar[k], xi = ai[k];
+  const T vr = xr * rr - xi * ri;
+  const T vi = xr * ri + xi * rr;
+  ar[k] = act ? vr : xr;
+  ai[k] = act ? vi : xi;
+  T lr = act ? vr : T(0), li = act ? vi : T(0);
+  pin(ar[k]);
+  pin(ai[k]);
+  pin(lr);
+  pin(li);
+#pragma unroll
+  for (int j0 = k + 1; j0 < N; j0 += kBcastChunk) {
+    __builtin_amdgcn_sched_barrier(0);
+    T ur[kBcastChunk], ui[kBcastChunk];
+#pragma unroll
+    for (int j = j0; j < j0 + kBcastChunk; ++j)
+      if (j < N) {
+        ur[j - j0] = Grp<64>::bcast(ar[j], plane);
+        ui[j - j0] = Grp<64>::bcast(ai[j], plane);
+      }
+#pragma unroll
+    for (int j = j0; j < j0 + kBcastChunk; ++j)
+      if (j < N) {
+        ar[j] = fma(li, ui[j - j0], fma(-lr, ur[j - j0], ar[j]));
+        ai[j] = fma(-li, ur[j - j0], fma(-lr, ui[j - j0], ai[j]));
+        pin(ar[j]);
+        pin(ai[j]);
+      }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+}
+
 template <int N, int G, int R, class T>
 __device__ __forceinline__ void lu_cplx_step(const int k, T (&ar)[R][N], T (&ai)[R][N], int (&pos)[R],
                                              Perm<N>& perm, T (&rdr)[R], T (&rdi)[R], int& info) {
   const int ln = Grp<G>::lane();
   int bkey = 0x7fffffff;
-  if constexpr (G == 64 && R == 1 && std::is_same<T, float>::value) {
-    bkey = pivot_key64(fabs(ar[0][k]) + fabs(ai[0][k]), (pos[0] << 8) | Rows<N, G, R>::row(ln, 0), pos[0] >= k);
-  } else {
-    T bv = T(-1);
+  T bv = T(-1);
 #pragma unroll
-    for (int q = 0; q < R; ++q) {
-      const bool act = pos[q] >= k;
-      const T v = fabs(ar[q][k]) + fabs(ai[q][k]);
-      const int key = (pos[q] << 8) | Rows<N, G, R>::row(ln, q);
-      const bool better = act && (v > bv || (v == bv && key < bkey));
-      bv = better ? v : bv;
-      bkey = better ? key : bkey;
-    }
-    group_argmax<G>(bv, bkey);
+  for (int q = 0; q < R; ++q) {
+    const bool act = pos[q] >= k;
+    const T v = fabs(ar[q][k]) + fabs(ai[q][k]);
+    const int key = (pos[q] << 8) | Rows<N, G, R>::row(ln, q);
+    const bool better = act && (v > bv || (v == bv && key < bkey));
+    bv = better ? v : bv;
+    bkey = better ? key : bkey;
   }
+  group_argmax<G>(bv, bkey);
   const int prow = bkey & 0xff;
   const int ppos = bkey >> 8;
   const int plane = prow % G;
@@ -618,11 +777,49 @@ __device__ __forceinline__ void lu_cplx(T (&ar)[R][N], T (&ai)[R][N], int (&pos)
   lu_init<N, G, R, T>(pos, rdr, info);
 #pragma unroll
   for (int q = 0; q < R; ++q) rdi[q] = T(0);
+  if constexpr (G == 64 && R == 1) {
+    Perm<N> pm = {};
+    int inf = 0;
 #pragma unroll
-  for (int k = 0; k < N; ++k) lu_cplx_step<N, G, R, T>(k, ar, ai, pos, perm, rdr, rdi, info);
+    for (int k = 0; k < N; ++k) wave_lu_cplx_step<N, T>(k, ar[0], ai[0], pos[0], pm, rdr[0], rdi[0], inf);
+    perm = pm;
+    info = inf;
+  } else {
+#pragma unroll
+    for (int k = 0; k < N; ++k) lu_cplx_step<N, G, R, T>(k, ar, ai, pos, perm, rdr, rdi, info);
+  }
 }
 
 // ---- triangular solves (dgetrs / zgetrs, nrhs = 1) ---------------------------
+// A solve's view of the row positions and of the pivot rows.  The rows that do
+// not take part in a step keep their right-hand side by a select on the
+// result; both the positions and (64-lane groups) the pivot rows, read into
+// scalar registers, are opaque to the compiler, so that no select, compare or
+// table entry looks invariant in the Newton loop: hoisted out of it, the
+// masked copies of all three factors alone needed as many registers as the
+// factors again, and every solve read them back from scratch.
+template <int N, int G, int R>
+struct SolveView {
+  int pos[R];
+  Perm<N> perm;
+  __device__ __forceinline__ SolveView(const int (&p)[R], const Perm<N>& pm) {
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      pos[q] = p[q];
+      __asm__ volatile("" : "+v"(pos[q]));
+    }
+#pragma unroll
+    for (int i = 0; i < (N + 3) / 4; ++i) {
+      if constexpr (G == 64) {
+        perm.w[i] = (uint32_t)__builtin_amdgcn_readfirstlane((int)pm.w[i]);
+        __asm__ volatile("" : "+s"(perm.w[i]));
+      } else {
+        perm.w[i] = pm.w[i];
+      }
+    }
+  }
+};
+
 // b[q] is the right-hand side of row r = row(ln, q); on return it holds
 // solution component r.  Forward then backward column-oriented substitution in
 // pivot order, as reference BLAS dtrsm does it; rows outside the current
@@ -633,7 +830,10 @@ __device__ __forceinline__ void fwd_real_step(const int k, const T (&a)[R][N], c
   const int prow = perm.get(k);
   const T yk = Grp<G>::bcast(sel<R>(b, prow / G), prow % G);
 #pragma unroll
-  for (int q = 0; q < R; ++q) b[q] = fma(-(pos[q] > k ? a[q][k] : T(0)), yk, b[q]);
+  for (int q = 0; q < R; ++q) {
+    const T v = fma(-a[q][k], yk, b[q]);
+    b[q] = pos[q] > k ? v : b[q];
+  }
 }
 
 template <int N, int G, int R, class T>
@@ -645,7 +845,8 @@ __device__ __forceinline__ void bwd_real_step(const int k, const T (&a)[R][N], c
   const T xk = Grp<G>::bcast(sel<R>(b, pq) * sel<R>(rd, pq), prow % G);
 #pragma unroll
   for (int q = 0; q < R; ++q) {
-    b[q] = fma(-((pos[q] >= 0 && pos[q] < k) ? a[q][k] : T(0)), xk, b[q]);
+    const T v = fma(-a[q][k], xk, b[q]);
+    b[q] = (unsigned)pos[q] < (unsigned)k ? v : b[q];  // (pos = -1: padding rows)
     x[q] = (Rows<N, G, R>::row(ln, q) == k) ? xk : x[q];
   }
 }
@@ -654,13 +855,14 @@ template <int N, int G, int R, class T>
 __device__ __forceinline__ void solve_real(const T (&a)[R][N], const int (&pos)[R],
                                            const Perm<N>& perm, const T (&rd)[R],
                                            T (&b)[R]) {
+  const SolveView<N, G, R> v(pos, perm);
 #pragma unroll
-  for (int k = 0; k < N; ++k) fwd_real_step<N, G, R, T>(k, a, pos, perm, b);
+  for (int k = 0; k < N; ++k) fwd_real_step<N, G, R, T>(k, a, v.pos, v.perm, b);
   T x[R];
 #pragma unroll
   for (int q = 0; q < R; ++q) x[q] = T(0);
 #pragma unroll
-  for (int k = N - 1; k >= 0; --k) bwd_real_step<N, G, R, T>(k, a, pos, perm, rd, b, x);
+  for (int k = N - 1; k >= 0; --k) bwd_real_step<N, G, R, T>(k, a, v.pos, v.perm, rd, b, x);
 #pragma unroll
   for (int q = 0; q < R; ++q) b[q] = x[q];
 }
@@ -675,11 +877,11 @@ __device__ __forceinline__ void fwd_cplx_step(const int k, const T (&ar)[R][N], 
 #pragma unroll
   for (int q = 0; q < R; ++q) {
     const bool act = pos[q] > k;
-    const T lr = act ? ar[q][k] : T(0), li = act ? ai[q][k] : T(0);
-    br[q] = fma(-lr, yr, br[q]);
-    br[q] = fma(li, yi, br[q]);
-    bi[q] = fma(-lr, yi, bi[q]);
-    bi[q] = fma(-li, yr, bi[q]);
+    const T lr = ar[q][k], li = ai[q][k];
+    const T vr = fma(li, yi, fma(-lr, yr, br[q]));
+    const T vi = fma(-li, yr, fma(-lr, yi, bi[q]));
+    br[q] = act ? vr : br[q];
+    bi[q] = act ? vi : bi[q];
   }
 }
 
@@ -696,12 +898,12 @@ __device__ __forceinline__ void bwd_cplx_step(const int k, const T (&ar)[R][N], 
   const T ki = Grp<G>::bcast(vr * di + vi * dr, pl);
 #pragma unroll
   for (int q = 0; q < R; ++q) {
-    const bool act = pos[q] >= 0 && pos[q] < k;
-    const T ur = act ? ar[q][k] : T(0), ui = act ? ai[q][k] : T(0);
-    br[q] = fma(-ur, kr, br[q]);
-    br[q] = fma(ui, ki, br[q]);
-    bi[q] = fma(-ur, ki, bi[q]);
-    bi[q] = fma(-ui, kr, bi[q]);
+    const bool act = (unsigned)pos[q] < (unsigned)k;
+    const T ur = ar[q][k], ui = ai[q][k];
+    const T vr2 = fma(ui, ki, fma(-ur, kr, br[q]));
+    const T vi2 = fma(-ui, kr, fma(-ur, ki, bi[q]));
+    br[q] = act ? vr2 : br[q];
+    bi[q] = act ? vi2 : bi[q];
     const bool mine = Rows<N, G, R>::row(ln, q) == k;
     xr[q] = mine ? kr : xr[q];
     xi[q] = mine ? ki : xi[q];
@@ -713,13 +915,14 @@ __device__ __forceinline__ void solve_cplx(const T (&ar)[R][N], const T (&ai)[R]
                                            const int (&pos)[R], const Perm<N>& perm,
                                            const T (&rdr)[R], const T (&rdi)[R],
                                            T (&br)[R], T (&bi)[R]) {
+  const SolveView<N, G, R> v(pos, perm);
 #pragma unroll
-  for (int k = 0; k < N; ++k) fwd_cplx_step<N, G, R, T>(k, ar, ai, pos, perm, br, bi);
+  for (int k = 0; k < N; ++k) fwd_cplx_step<N, G, R, T>(k, ar, ai, v.pos, v.perm, br, bi);
   T xr[R], xi[R];
 #pragma unroll
   for (int q = 0; q < R; ++q) { xr[q] = T(0); xi[q] = T(0); }
 #pragma unroll
-  for (int k = N - 1; k >= 0; --k) bwd_cplx_step<N, G, R, T>(k, ar, ai, pos, perm, rdr, rdi, br, bi, xr, xi);
+  for (int k = N - 1; k >= 0; --k) bwd_cplx_step<N, G, R, T>(k, ar, ai, v.pos, v.perm, rdr, rdi, br, bi, xr, xi);
 #pragma unroll
   for (int q = 0; q < R; ++q) { br[q] = xr[q]; bi[q] = xi[q]; }
 }
