@@ -23,6 +23,7 @@
 
 #include <string.h>
 
+#include <algorithm>
 #include <string>
 #include <vector>
 
@@ -35,6 +36,12 @@ constexpr int kKinMaxReactions = 4096;
 // Jacobian's d wdot / d C accumulation
 constexpr int kKinRhsBatch = 8;
 constexpr int kKinJacBatch = 8;
+// Reactions a lane evaluates side by side in dydt.  A 64-lane group has the
+// registers (one wave per SIMD) and no other wave to fill the waits: two at a
+// time take the 54-state FP32-factor launch (65536 conditions) from 165.3 to
+// 162.1 ms.  16-lane groups run two waves per SIMD on half the registers: two at a
+// time spill (262144 14-state conditions, FP64: 30.0 -> 37.7 ms).
+constexpr int rxn_unroll(int G) { return G == 64 ? 2 : 1; }
 
 // *p += v in LDS, no return value: the LDS applies a wavefront's operations
 // in issue order, so successive adds to one address keep their order.
@@ -55,22 +62,39 @@ constexpr double kKinTmax = 1.0e4;
 constexpr double kKinSmin = 1.0e-3;
 constexpr double kKinCpmin = 1.0;
 
+// One reaction as the rate loop reads it, from global memory (each lane only
+// its own reactions): rate parameters, net mole change, and the byte offsets of
+// its six slots' species in the group's (C, g/RT) pairs -- reactants 0..2,
+// products 3..5, empty slots the dummy species NS (C = 1, g = h = 0), so the
+// loop has no test per slot.
+struct alignas(16) KinReaction {
+  double lnA, beta, EaR, dnu;
+  uint16_t off[6];
+  uint16_t pad[2];
+};
+static_assert(sizeof(KinReaction) == 48, "three 16-byte loads");
+
 // Device view of a network: one packed blob (built by KineticsHost).  Its
-// first lds_bytes (the tables read at data-dependent indices) are copied by
-// every block into the front of its LDS at kernel start; the per-reaction rate
-// parameters, which each lane reads only for its own reactions, stay in global
-// memory (L2 resident).  Byte offsets:
-//   [off_invW] double invW[ns]      [off_W] double W[ns]
-//   [off_th]   double thermo[5 ns]  [off_sl] uint64 slots[nr] (byte a = species of slot a, 0xff = empty)
+// first lds_bytes (the tables that are read at data-dependent indices by the
+// Jacobian) are copied by every block into the front of its LDS at kernel
+// start; what a lane reads only for its own species or reactions stays in
+// global memory (cache resident).  Species tables carry the dummy species NS.
+// Byte offsets:
+//   [off_invW] double invW[ns + 1]  [off_sl] uint64 slots[nr] (byte a = species of slot a, ns = empty)
 //   [off_co]   int csr_off[ns + 1]  [off_ce] int csr[nnz] = (reaction << 8) | (nu & 0xff)
 //   ---- end of the LDS part (lds_bytes) ----
-//   [off_rc]   double rc[3 nr] (lnA, beta, EaR)
+//   [off_W]    double W[ns + 1]     [off_th] double thermo[5 (ns + 1)]
+//   [off_rx]   KinReaction[nr]
+//   [off_el]   the incidence list once more, for dydt: ell_batches batches of
+//              kKinRhsBatch entries for every species (int ell[batch][half][ns + 1][4]),
+//              entry = (byte offset of the reaction's q in the group's LDS << 16) | (nu & 0xffff);
+//              lists end in entries that add 0 x 0
 struct KinParams {
   const double* blob;  // device copy
   int blob_bytes;      // multiple of 16
   int lds_bytes;       // multiple of 16, the LDS-resident prefix
   int ns, nr, nnz;
-  int off_invW, off_W, off_th, off_rc, off_sl, off_co, off_ce;
+  int off_invW, off_W, off_th, off_sl, off_co, off_ce, off_rx, off_el, ell_batches;
 };
 
 template <int NTOT>
@@ -95,12 +119,12 @@ struct MechKinetics {
   // Callbacks: dydt returns the rows a lane owns; jacob writes the dense
   // Jacobian into the group's LDS (kJacInLds), where the integrator keeps it.
   //
-  // per group: C, gRT, hR, cpR [NS each]; kf, kr, q, qT [nr each]; the
+  // per group: (C, gRT) pairs, hR, cpR [NS + 1 each]; kf, kr, q, qT [nr each]; the
   // Jacobian buffer [N*N] (d wdot / d C rows while the Jacobian is assembled,
   // then the parked Jacobian); optionally a scratch [N*N] for integrators that
   // transpose their factors through LDS.
   __host__ __device__ static size_t group_doubles(int nr, bool scratch) {
-    return (size_t)4 * NS + (size_t)4 * nr + (kLarge ? 0 : (size_t)(scratch ? 2 : 1) * N * N);
+    return (size_t)4 * (NS + 1) + (size_t)4 * nr + (kLarge ? 0 : (size_t)(scratch ? 2 : 1) * N * N);
   }
   static size_t lds_bytes(const Params& p, int groups, bool scratch) {
     return (size_t)p.lds_bytes + groups * group_doubles(p.nr, scratch) * sizeof(double);
@@ -116,16 +140,16 @@ struct MechKinetics {
   }
 
   struct Ctx {
-    int nr;
+    int nr, ell_batches;
     const double* invW;
     const double* W;
     const double* thermo;
-    const double* rc;
+    const KinReaction* rx;
+    const int4* ell;
     const unsigned long long* slots;
     const int* csr_off;
     const int* csr;
-    double* C;
-    double* gRT;
+    double2* cg;  // (C, g/RT) per species
     double* hR;
     double* cpR;
     double* kf;
@@ -139,20 +163,22 @@ struct MechKinetics {
     __device__ Ctx(const Params& pp, int g, double* lds, bool with_scratch)
         : Ctx(pp, lds, lds + pp.lds_bytes / 8 + (size_t)g * group_doubles(pp.nr, with_scratch), with_scratch) {}
     // tables at `tables`, the group's buffers at `group` (group_doubles(nr, with_scratch) doubles)
-    __device__ Ctx(const Params& pp, const double* tables, double* group, bool with_scratch) : nr(pp.nr) {
+    __device__ Ctx(const Params& pp, const double* tables, double* group, bool with_scratch)
+        : nr(pp.nr), ell_batches(pp.ell_batches) {
       const char* t = reinterpret_cast<const char*>(tables);
+      const char* gl = reinterpret_cast<const char*>(pp.blob);
       invW = reinterpret_cast<const double*>(t + pp.off_invW);
-      W = reinterpret_cast<const double*>(t + pp.off_W);
-      thermo = reinterpret_cast<const double*>(t + pp.off_th);
-      rc = reinterpret_cast<const double*>(reinterpret_cast<const char*>(pp.blob) + pp.off_rc);
+      W = reinterpret_cast<const double*>(gl + pp.off_W);
+      thermo = reinterpret_cast<const double*>(gl + pp.off_th);
+      rx = reinterpret_cast<const KinReaction*>(gl + pp.off_rx);
+      ell = reinterpret_cast<const int4*>(gl + pp.off_el);
       slots = reinterpret_cast<const unsigned long long*>(t + pp.off_sl);
       csr_off = reinterpret_cast<const int*>(t + pp.off_co);
       csr = reinterpret_cast<const int*>(t + pp.off_ce);
       double* b = group;
-      C = b; b += NS;
-      gRT = b; b += NS;
-      hR = b; b += NS;
-      cpR = b; b += NS;
+      cg = reinterpret_cast<double2*>(b); b += 2 * (NS + 1);
+      hR = b; b += NS + 1;
+      cpR = b; b += NS + 1;
       kf = b; b += pp.nr;
       kr = b; b += pp.nr;
       q = b; b += pp.nr;
@@ -180,168 +206,173 @@ struct MechKinetics {
     double T, lnT, iT, S, Ctot, cpm, dcpm;
   };
 
+  // species of row q of this lane; rows that hold none (the temperature row,
+  // padding rows) take the dummy species, so that no step below is conditional
+  template <int G>
+  __device__ __forceinline__ static int species(int q) {
+    const int r = Grp<G>::lane() + G * q;
+    return r >= 1 && r < N ? r - 1 : NS;
+  }
+
   // Shared prologue: T, thermo of owned species (to LDS), mixture sums and
   // concentrations (to LDS).
-  template <int G, int R>
+  template <int G, int R, bool JAC>
   __device__ __forceinline__ static void prologue(Ctx& c, double P, const double (&y)[R], Mix& m) {
-    const int ln = Grp<G>::lane();
+    double a0[R], a1[R], a2[R], bh[R], bs[R], iw[R], yv[R];
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      const int s = species<G>(q);
+      const double* a = c.thermo + 5 * s;
+      a0[q] = a[0];
+      a1[q] = a[1];
+      a2[q] = a[2];
+      bh[q] = a[3];
+      bs[q] = a[4];
+      iw[q] = c.invW[s];
+      yv[q] = s < NS ? y[q] : 0.0;
+    }
     const double T = fmin(fmax(Grp<G>::bcast(y[0], 0), kKinTmin), kKinTmax);
     const double lnT = log(T);
     const double iT = 1.0 / T;
     double Sp = 0.0, cpp = 0.0, dcp = 0.0;
+    double g[R];
 #pragma unroll
     for (int q = 0; q < R; ++q) {
-      const int r = ln + G * q;
-      if (r >= 1 && r < N) {
-        const int s = r - 1;
-        const double* a = c.thermo + 5 * s;
-        const double a0 = a[0], a1 = a[1], a2 = a[2], bh = a[3], bs = a[4];
-        const double cp = a0 + a1 * T + a2 * T * T;
-        const double h = a0 * T + a1 * T * T * 0.5 + a2 * T * T * T * (1.0 / 3.0) + bh;
-        const double sR = a0 * lnT + a1 * T + a2 * T * T * 0.5 + bs;
-        c.cpR[s] = cp;
-        c.hR[s] = h;
-        c.gRT[s] = h * iT - sR;
-        const double iw = c.invW[s];
-        Sp += y[q] * iw;
-        cpp += y[q] * cp * iw;
-        dcp += y[q] * (a1 + 2 * a2 * T) * iw;
-      }
+      const int s = species<G>(q);
+      const double cp = a0[q] + a1[q] * T + a2[q] * T * T;
+      const double h = a0[q] * T + a1[q] * T * T * 0.5 + a2[q] * T * T * T * (1.0 / 3.0) + bh[q];
+      const double sR = a0[q] * lnT + a1[q] * T + a2[q] * T * T * 0.5 + bs[q];
+      if (JAC) c.cpR[s] = cp;
+      c.hR[s] = h;
+      g[q] = h * iT - sR;
+      Sp += yv[q] * iw[q];
+      cpp += yv[q] * cp * iw[q];
+      dcp += yv[q] * (a1[q] + 2 * a2[q] * T) * iw[q];
     }
     m.T = T;
     m.lnT = lnT;
     m.iT = iT;
-    m.S = fmax(Grp<G>::sum(Sp), kKinSmin);
-    m.cpm = fmax(kKinR * Grp<G>::sum(cpp), kKinCpmin);
-    m.dcpm = kKinR * Grp<G>::sum(dcp);
+    Grp<G>::sum2(Sp, cpp);
+    m.S = fmax(Sp, kKinSmin);
+    m.cpm = fmax(kKinR * cpp, kKinCpmin);
+    m.dcpm = JAC ? kKinR * Grp<G>::sum(dcp) : 0.0;
     m.Ctot = (1e-6 / kKinR) * P * iT;
     const double cs = m.Ctot / m.S;
 #pragma unroll
     for (int q = 0; q < R; ++q) {
-      const int r = ln + G * q;
-      if (r >= 1 && r < N) {
-        const int s = r - 1;
-        c.C[s] = cs * (y[q] * c.invW[s]);
-      }
+      const int s = species<G>(q);
+      c.cg[s] = double2{s < NS ? cs * (yv[q] * iw[q]) : 1.0, g[q]};
     }
     group_lds_sync();
   }
 
-  // Rate constants and rates of progress of the reactions this lane handles.
-  template <int G, bool JAC>
+  // Rate constants and rates of progress of the reactions this lane handles,
+  // U at a time (independent chains through the exponentials and the gathers
+  // of each other); the records of the next U are fetched one pass ahead.
+  // Passes beyond nr repeat the last reaction.  Bound by issue and by the
+  // exponentials' dependent chains; the dummy species and the precomputed
+  // offsets took a pass from ~160 to ~90 instructions.
+  template <int G, bool JAC, int U>
   __device__ __forceinline__ static void reactions(Ctx& c, const Mix& m) {
     const int ln = Grp<G>::lane();
     const double lnC0 = kKinLnC0R - m.lnT;  // ln(1e-6 P_atm / (R T))
     const double lnTr = m.lnT - kKinLnTref;
     const double iT = m.iT;
-    // rate parameters (global memory) and slot words (LDS) are fetched one
-    // reaction ahead; the species data of a reaction's six slots are
-    // gathered together (in-bounds index, then a select) before any is used
-    double nlnA = 0.0, nbeta = 0.0, nEaR = 0.0;
-    unsigned long long nsw = ~0ull;
-    if (ln < c.nr) {
-      nlnA = c.rc[3 * ln];
-      nbeta = c.rc[3 * ln + 1];
-      nEaR = c.rc[3 * ln + 2];
-      nsw = c.slots[ln];
-    }
+    const int last = c.nr - 1;
+    const char* cg = reinterpret_cast<const char*>(c.cg);
+    KinReaction nx[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) nx[u] = c.rx[min(ln + u * G, last)];
 #pragma unroll 1
-    for (int j = ln; j < c.nr; j += G) {
-      const unsigned long long sw = nsw;
-      const double lnA = nlnA, beta = nbeta, EaR = nEaR;
-      if (j + G < c.nr) {
-        nlnA = c.rc[3 * (j + G)];
-        nbeta = c.rc[3 * (j + G) + 1];
-        nEaR = c.rc[3 * (j + G) + 2];
-        nsw = c.slots[j + G];
-      }
-      double gv[6], hv[6], cv[6];
+    for (int j0 = 0; j0 < c.nr; j0 += U * G) {
+      KinReaction x[U];
+      double2 v[U][6];
 #pragma unroll
-      for (int a = 0; a < 6; ++a) {
-        const int s = (int)((sw >> (8 * a)) & 0xffu);
-        const int si = s != 0xff ? s : 0;
-        gv[a] = c.gRT[si];
-        if (JAC) hv[a] = c.hR[si];
-        cv[a] = c.C[si];
-      }
-      double sum_nu_g = 0.0, sum_nu_h = 0.0;
-      int dnu = 0;
-      double pf = 1.0, pr = 1.0;
+      for (int u = 0; u < U; ++u) x[u] = nx[u];
 #pragma unroll
-      for (int a = 0; a < 6; ++a) {
-        const int s = (int)((sw >> (8 * a)) & 0xffu);
-        if (s != 0xff) {
-          if (a < 3) {
-            sum_nu_g -= gv[a];
-            if (JAC) sum_nu_h -= hv[a];
-            dnu -= 1;
-            pf *= cv[a];
-          } else {
-            sum_nu_g += gv[a];
-            if (JAC) sum_nu_h += hv[a];
-            dnu += 1;
-            pr *= cv[a];
-          }
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int a = 0; a < 6; ++a) v[u][a] = *reinterpret_cast<const double2*>(cg + x[u].off[a]);
+      if (j0 + U * G < c.nr) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) nx[u] = c.rx[min(j0 + ln + (U + u) * G, last)];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int j = min(j0 + ln + u * G, last);
+        const double sum_nu_g = 0.0 - v[u][0].y - v[u][1].y - v[u][2].y + v[u][3].y + v[u][4].y + v[u][5].y;
+        double pf = v[u][0].x * v[u][1].x * v[u][2].x;
+        double pr = v[u][3].x * v[u][4].x * v[u][5].x;
+        const double lnkf = x[u].lnA + x[u].beta * lnTr - x[u].EaR * iT;
+        const double lnKc = -sum_nu_g + x[u].dnu * lnC0;
+        const double kf = exp(lnkf);
+        const double kr = exp(lnkf - lnKc);
+        pf *= kf;
+        pr *= kr;
+        c.q[j] = pf - pr;
+        if (JAC) {
+          double h[6];
+#pragma unroll
+          for (int a = 0; a < 6; ++a) h[a] = c.hR[x[u].off[a] / 16];
+          const double sum_nu_h = 0.0 - h[0] - h[1] - h[2] + h[3] + h[4] + h[5];
+          const double dlnkf = (x[u].beta + x[u].EaR * iT) * iT;
+          const double dlnkr = dlnkf - (sum_nu_h * iT - x[u].dnu) * iT;
+          c.qT[j] = pf * dlnkf - pr * dlnkr;
+          c.kf[j] = kf;
+          c.kr[j] = kr;
         }
-      }
-      const double lnkf = lnA + beta * lnTr - EaR * iT;
-      const double lnKc = -sum_nu_g + dnu * lnC0;
-      const double kf = exp(lnkf);
-      const double kr = exp(lnkf - lnKc);
-      pf *= kf;
-      pr *= kr;
-      c.q[j] = pf - pr;
-      if (JAC) {
-        const double dlnkf = (beta + EaR * iT) * iT;
-        const double dlnkr = dlnkf - (sum_nu_h * iT - dnu) * iT;
-        c.qT[j] = pf * dlnkf - pr * dlnkr;
-        c.kf[j] = kf;
-        c.kr[j] = kr;
       }
     }
     group_lds_sync();
   }
 
+  // Bound at one wave per SIMD by issue and exposed LDS round trips.  Without
+  // per-slot tests, with the species' lists read from global memory as whole
+  // batches (5 instead of 13 instructions per entry) and with nothing
+  // conditional, states bit-identical: 32768 54-state conditions of one global
+  // step FP64 117.1 -> 106.7 ms, 65536 with FP32 factors 185.3 -> 162.1 ms, 262144
+  // 14-state conditions of two steps 35.2 -> 30.0 ms.
   template <int G, int R>
   __device__ __forceinline__ static void dydt(Ctx& c, double, double P, const double (&y)[R],
                                               double (&f)[R]) {
     const int ln = Grp<G>::lane();
     Mix m;
-    prologue<G, R>(c, P, y, m);
-    reactions<G, false>(c, m);
+    prologue<G, R, false>(c, P, y, m);
+    reactions<G, false, rxn_unroll(G)>(c, m);
     const double D = m.S / m.Ctot;
+    const char* base = reinterpret_cast<const char*>(c.cg);
     double Qp = 0.0;
 #pragma unroll
     for (int q = 0; q < R; ++q) {
-      const int r = ln + G * q;
-      f[q] = 0.0;
-      if (r >= 1 && r < N) {
-        const int s = r - 1;
-        // incidence list in batches: the batch's entries, then its rates,
-        // are fetched before any is summed (two LDS round trips per batch
-        // instead of two per entry); the sum keeps the list order
-        double w = 0.0;
-        const int e1 = c.csr_off[s + 1];
+      // incidence list in batches of eight, all lists as long as the longest:
+      // the batch after this one is fetched while this one's rates are summed
+      // in list order; entries beyond a list's end add an exact zero
+      const int s = species<G>(q);
+      const int4* e = c.ell + s;
+      int4 n0 = e[0], n1 = e[NS + 1];
+      double w = 0.0;
 #pragma unroll 1
-        for (int e = c.csr_off[s]; e < e1; e += kKinRhsBatch) {
-          int ce[kKinRhsBatch];
-          double qv[kKinRhsBatch];
+      for (int b = 0; b < c.ell_batches; ++b) {
+        const int ce[8] = {n0.x, n0.y, n0.z, n0.w, n1.x, n1.y, n1.z, n1.w};
+        double qv[8];
 #pragma unroll
-          for (int i = 0; i < kKinRhsBatch; ++i) ce[i] = c.csr[min(e + i, e1 - 1)];
-#pragma unroll
-          for (int i = 0; i < kKinRhsBatch; ++i) qv[i] = c.q[ce[i] >> 8];
-#pragma unroll
-          for (int i = 0; i < kKinRhsBatch; ++i)
-            if (e + i < e1) w += (double)(signed char)(ce[i] & 0xff) * qv[i];
+        for (int i = 0; i < 8; ++i) qv[i] = *reinterpret_cast<const double*>(base + ((unsigned)ce[i] >> 16));
+        if (b + 1 < c.ell_batches) {
+          e += 2 * (NS + 1);
+          n0 = e[0];
+          n1 = e[NS + 1];
         }
-        f[q] = c.W[s] * w * D;
-        Qp += c.hR[s] * w;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) w += (double)(short)ce[i] * qv[i];
       }
+      f[q] = s < NS ? c.W[s] * w * D : 0.0;
+      Qp += c.hR[s] * w;
     }
     const double Q = kKinR * Grp<G>::sum(Qp);
+    const double fT = -Q * D / m.cpm;
 #pragma unroll
     for (int q = 0; q < R; ++q)
-      if (ln + G * q == 0) f[q] = -Q * D / m.cpm;
+      if (ln + G * q == 0) f[q] = fT;
     group_lds_sync();  // LDS is reused by the next evaluation
   }
 
@@ -361,8 +392,8 @@ struct MechKinetics {
     }
     const int ln = Grp<G>::lane();
     Mix m;
-    prologue<G, R>(c, P, y, m);
-    reactions<G, true>(c, m);
+    prologue<G, R, true>(c, P, y, m);
+    reactions<G, true, 1>(c, m);
     const double S = m.S, Ctot = m.Ctot, iT = m.iT;
     const double D = S / Ctot;
     double Qp = 0.0, dQp = 0.0;
@@ -410,8 +441,7 @@ struct MechKinetics {
 #pragma unroll
             for (int a = 0; a < 6; ++a) {
               const int sa = (int)((swv[i] >> (8 * a)) & 0xffu);
-              const double x = c.C[sa != 0xff ? sa : 0];
-              cv[i][a] = sa != 0xff ? x : 1.0;
+              cv[i][a] = c.cg[sa].x;  // 1 for an empty slot
             }
 #pragma unroll
           for (int i = 0; i < B; ++i) {
@@ -423,7 +453,7 @@ struct MechKinetics {
 #pragma unroll
               for (int b = 0; b < 6; ++b) {
                 const int sb = (int)((swv[i] >> (8 * b)) & 0xffu);
-                if (sb != 0xff) {
+                if (sb != NS) {
                   double v = b < 3 ? kfj : krj;
                   const int lo = b < 3 ? 0 : 3;
 #pragma unroll
@@ -440,7 +470,7 @@ struct MechKinetics {
 #pragma unroll
         for (int i = 0; i < NS; ++i) {
           jr[q][i] = row[i];
-          rs += jr[q][i] * c.C[i];
+          rs += jr[q][i] * c.cg[i].x;
         }
         rsv[q] = rs;
         wv[q] = w;
@@ -505,8 +535,8 @@ struct MechKinetics {
     constexpr int LD = kJacLd;
     const int ln = Grp<G>::lane();
     Mix m;
-    prologue<G, R>(c, P, y, m);
-    reactions<G, true>(c, m);
+    prologue<G, R, true>(c, P, y, m);
+    reactions<G, true, 1>(c, m);
     const double S = m.S, Ctot = m.Ctot, iT = m.iT;
     const double D = S / Ctot;
     double Qp = 0.0, dQp = 0.0, HRp = 0.0;
@@ -535,12 +565,12 @@ struct MechKinetics {
 #pragma unroll
           for (int a = 0; a < 6; ++a) {
             sp[a] = (int)((sw >> (8 * a)) & 0xffu);
-            cv[a] = sp[a] != 0xff ? c.C[sp[a]] : 1.0;
+            cv[a] = c.cg[sp[a]].x;  // 1 for an empty slot
           }
           const double kfj = nu * c.kf[j], krj = -nu * c.kr[j];
 #pragma unroll
           for (int b = 0; b < 6; ++b) {
-            if (sp[b] != 0xff) {
+            if (sp[b] != NS) {
               double v = b < 3 ? kfj : krj;
               const int lo = b < 3 ? 0 : 3;
 #pragma unroll
@@ -552,7 +582,7 @@ struct MechKinetics {
         }
         double rs = 0.0;
 #pragma unroll 4
-        for (int i = 0; i < NS; ++i) rs += row[(size_t)i * LD] * c.C[i];
+        for (int i = 0; i < NS; ++i) rs += row[(size_t)i * LD] * c.cg[i].x;
         rsv[q] = rs;
         wv[q] = w;
         wTv[q] = wT;
@@ -693,7 +723,7 @@ struct KineticsHost {
       unsigned long long w = 0;
       for (int a = 0; a < 6; ++a) {
         const int sp = slots[6 * j + a];
-        w |= (unsigned long long)(sp < 0 ? 0xff : sp) << (8 * a);
+        w |= (unsigned long long)(sp < 0 ? ns : sp) << (8 * a);
       }
       sl[j] = w;
     }
@@ -702,14 +732,46 @@ struct KineticsHost {
     dev.ns = ns;
     dev.nr = nr;
     dev.nnz = nnz;
-    dev.off_invW = section(invW.data(), ns * sizeof(double));
-    dev.off_W = section(W.data(), ns * sizeof(double));
-    dev.off_th = section(thermo.data(), 5 * (size_t)ns * sizeof(double));
+    // species tables with the dummy species (all zero) at the end
+    std::vector<double> invWd(invW), Wd(W), thd(thermo);
+    invWd.push_back(0.0);
+    Wd.push_back(0.0);
+    thd.resize(5 * ((size_t)ns + 1), 0.0);
+    std::vector<KinReaction> rx(nr);
+    for (int j = 0; j < nr; ++j) {
+      KinReaction& r = rx[j];
+      r = KinReaction{};
+      r.lnA = rc[3 * j];
+      r.beta = rc[3 * j + 1];
+      r.EaR = rc[3 * j + 2];
+      for (int a = 0; a < 6; ++a) {
+        const int sp = slots[6 * j + a];
+        if (sp >= 0) r.dnu += a < 3 ? -1.0 : 1.0;
+        r.off[a] = (uint16_t)(16 * (sp < 0 ? ns : sp));
+      }
+    }
+    // dydt's incidence list: every species as many whole batches as the longest
+    static_assert(kKinRhsBatch == 8, "two int4 per batch");
+    int longest = 0;
+    for (int s = 0; s < ns; ++s) longest = std::max(longest, csr_off[s + 1] - csr_off[s]);
+    dev.ell_batches = std::max(1, (longest + 7) / 8);
+    const int zero = 8 * (3 * (ns + 1) - 1), q0 = 8 * (4 * (ns + 1) + 2 * nr);
+    std::vector<int> el((size_t)dev.ell_batches * 2 * (ns + 1) * 4, (int)((unsigned)zero << 16));
+    for (int s = 0; s < ns; ++s)
+      for (int e = csr_off[s]; e < csr_off[s + 1]; ++e) {
+        const int i = e - csr_off[s];
+        el[(((size_t)(i / 4)) * (ns + 1) + s) * 4 + i % 4] =
+            (int)(((unsigned)(q0 + 8 * csr_rxn[e]) << 16) | ((unsigned)csr_nu[e] & 0xffffu));
+      }
+    dev.off_invW = section(invWd.data(), invWd.size() * sizeof(double));
     dev.off_sl = section(sl.data(), (size_t)nr * sizeof(unsigned long long));
     dev.off_co = section(csr_off.data(), (size_t)(ns + 1) * sizeof(int));
     dev.off_ce = section(ce.data(), (size_t)ce.size() * sizeof(int));
     dev.lds_bytes = (int)blob.size();
-    dev.off_rc = section(rc.data(), 3 * (size_t)nr * sizeof(double));
+    dev.off_W = section(Wd.data(), Wd.size() * sizeof(double));
+    dev.off_th = section(thd.data(), thd.size() * sizeof(double));
+    dev.off_rx = section(rx.data(), rx.size() * sizeof(KinReaction));
+    dev.off_el = section(el.data(), el.size() * sizeof(int));
     dev.blob_bytes = (int)blob.size();
     if (hipMalloc(&dmem, blob.size()) != hipSuccess) {
       *msg = "hipMalloc failed for kinetics tables";

@@ -175,6 +175,9 @@ struct Grp {
   // Butterfly all-reduce: partners add the same two operands, so every lane
   // of the group ends with a bit-identical result.
   __device__ __forceinline__ static double sum(double v);
+  // two sums side by side: the same operations as two calls of sum, their
+  // dependent chains overlapped
+  __device__ __forceinline__ static void sum2(double& a, double& b);
 };
 
 // Row ownership helpers.
@@ -484,6 +487,31 @@ __device__ __forceinline__ double Grp<G>::sum(double v) {
     for (int m = 1; m < G; m <<= 1) v += xor_(v, m);
   }
   return v;
+}
+
+template <int G>
+__device__ __forceinline__ void Grp<G>::sum2(double& a, double& b) {
+  if constexpr (G == 16 || G == 64) {
+    double x = dpp_t<kDppXor1>(a), z = dpp_t<kDppXor1>(b);
+    a += x;
+    b += z;
+    x = dpp_t<kDppXor2>(a), z = dpp_t<kDppXor2>(b);
+    a += x;
+    b += z;
+    x = dpp_t<kDppHalfMirror>(a), z = dpp_t<kDppHalfMirror>(b);
+    a += x;
+    b += z;
+    x = dpp_t<kDppMirror>(a), z = dpp_t<kDppMirror>(b);
+    a += x;
+    b += z;
+    if constexpr (G == 64) {
+      a = (bcast(a, 0) + bcast(a, 16)) + (bcast(a, 32) + bcast(a, 48));
+      b = (bcast(b, 0) + bcast(b, 16)) + (bcast(b, 32) + bcast(b, 48));
+    }
+  } else {
+    a = sum(a);
+    b = sum(b);
+  }
 }
 
 // ---- real LU (dgetf2 semantics, implicit interchanges) ---------------------
