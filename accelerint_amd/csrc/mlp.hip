@@ -2,16 +2,27 @@
 // network's host-side owner (see mlp.hpp).  No counterpart in the reference.
 //
 // Training: mean squared error over normalized stage targets, Adam, batches of
-// B samples (B a multiple of 16).  Every matrix product (forward and backward)
-// is one call of k_mlp_gemm: a 16x16 output tile per wavefront, operands read
-// as FP32 from memory with arbitrary strides (transposes are stride choices),
-// rounded to BF16 (nearest even) in registers, accumulated in FP32.
+// B samples (B a multiple of 16).  Two kernels per batch: k_mlp_rows runs the
+// forward pass and the activations' gradients of 16 samples per block, row
+// local from the gathered sample to dZ1; k_mlp_weights forms one 16x16 tile of
+// a weight gradient per wavefront (or 16 bias gradients) over the whole batch
+// and applies Adam to it at once.  Matrix operands are rounded to BF16 (nearest
+// even) and accumulated in FP32 by v_mfma_f32_16x16x16_bf16, 16 values of the
+// summed index per instruction in ascending order.
+//
+// What bounds it: launches and the latency of a short dependent chain -- a batch
+// of 512 is 0.14 GFLOP and ~2 MB of traffic.  As one kernel per product and
+// elementwise pass with the loss read back after every batch (17 launches, a copy
+// and a device synchronization) a batch took 340 us; it takes 22 us now (two
+// epochs of 32768 samples from host arrays: 44.0 -> 4.3 ms, parameters and losses
+// bit-identical).
 #include <hip/hip_runtime.h>
 
 #include <math.h>
 #include <stdio.h>
 #include <string.h>
 
+#include <algorithm>
 #include <cmath>
 #include <random>
 #include <string>
@@ -22,109 +33,332 @@
 
 namespace acc {
 
-// C[M x N] (+)= A'[M x K] * B'[K x N] with A'(m, k) = A[m*sam + k*sak] and
-// B'(k, n) = B[k*sbk + n*sbn]; M, N, K multiples of 16.  4 waves per block.
-__global__ __launch_bounds__(256) void k_mlp_gemm(int M, int N, int K, const float* __restrict__ A, int sam,
-                                                  int sak, const float* __restrict__ B, int sbk, int sbn,
-                                                  float* __restrict__ C, int ldc, int accumulate) {
-  const int wave = blockIdx.x * 4 + (int)(threadIdx.x >> 6);
+// Device buffers of one batch (B samples, KT = B / 16 row tiles).  "Fragments"
+// hold BF16 matrix tiles as the MFMA operands want them with the samples as the
+// summed index: tile (row tile kt, column tile ct) lane l holds
+// M[16 kt + 4 (l / 16) + i][16 ct + l % 16], i = 0..3, at ((ct * KT + kt) * 64 + l).
+// That is also the layout of an MFMA result, so k_mlp_rows stores its result
+// registers as they are and k_mlp_weights streams them without a transpose.
+struct MlpBatch {
+  const float* x;    // samples, row stride `in`
+  const float* t;    // targets, row stride `out` (null: forward only)
+  const int* idx;    // sample rows of the batch (null: 0, 1, ...)
+  int in, inp, out, outp, rows;
+  // weights: BF16 B-operand tiles of W1, W2, W3 and of W2^T, W3^T; FP32 biases
+  const uint16_t *w1, *w2, *w3, *w2t, *w3t;
+  const float *b1, *b2, *b3;
+  // results
+  float* y;          // [rows][out] (forward only)
+  double* loss;      // squared error per row tile
+  mlp_bf16x4 *fx, *fa1, *fa2, *fdy, *fdz2, *fdz1;  // fragments
+  float *dy, *dz2, *dz1;                           // FP32 row-major (bias gradients)
+};
+
+constexpr int kMlpPad = 8;  // BF16 values between LDS rows: 16-byte rows, no bank pattern
+
+// Operand tiles (0 .. kts - 1, kts <= KTS) of column tile nt of a weight matrix,
+// in registers.
+template <int KTS>
+struct MlpW {
+  mlp_bf16x4 b[KTS];
+  __device__ __forceinline__ void load(const uint16_t* W, int nt, int kts) {
+    const mlp_bf16x4* p = reinterpret_cast<const mlp_bf16x4*>(W) + (size_t)nt * kts * 64 + (threadIdx.x & 63);
+#pragma unroll
+    for (int kt = 0; kt < KTS; ++kt)
+      if (kt < kts) b[kt] = p[(size_t)kt * 64];
+  }
+};
+// D tile (16 samples x 16 columns) of A B: A from LDS rows (BF16, leading
+// dimension lda).
+template <int KTS>
+__device__ __forceinline__ mlp_f32x4 mlp_tile(const uint16_t* A, int lda, const MlpW<KTS>& w, int kts) {
   const int l = (int)(threadIdx.x & 63);
-  const int tiles_n = N / 16;
-  const int tm = wave / tiles_n, tn = wave % tiles_n;
-  if (tm >= M / 16) return;  // whole waves only
-  const int m = tm * 16 + (l & 15), n = tn * 16 + (l & 15), kq = 4 * (l >> 4);
+  const uint16_t* a = A + (l & 15) * lda + 4 * (l >> 4);
   mlp_f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
-  for (int k0 = 0; k0 < K; k0 += 16) {
-    mlp_bf16x4 a, b;
+#pragma unroll
+  for (int kt = 0; kt < KTS; ++kt)
+    if (kt < kts)
+      acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(*reinterpret_cast<const mlp_bf16x4*>(a + 16 * kt), w.b[kt], acc,
+                                                      0, 0, 0);
+  return acc;
+}
+
+// Forward pass and (TRAIN) backward pass to dZ1 of 16 samples per block, eight
+// wavefronts: wavefront w owns hidden columns 16 w .. 16 w + 15 of both hidden
+// layers -- its pre-activations stay in registers from the forward to the
+// backward pass -- and output column tiles w and w + 8.  Activations pass
+// between layers through LDS as BF16.  The weights were last written by other
+// XCDs' compute units, so every first touch costs a trip past the L2; all of a
+// wavefront's operand tiles, biases and targets are therefore loaded into
+// registers up front, where one such latency covers them together (loaded
+// layer by layer the kernel took 19.2 us for 512 samples of a 54-state network,
+// now 15.0 us).
+template <bool TRAIN>
+__global__ __launch_bounds__(512) void k_mlp_rows(MlpBatch m) {
+  constexpr int H = kMlpHidden, HT = H / 16, LX = 64 + kMlpPad, LH = H + kMlpPad, LY = 192 + kMlpPad;
+  __shared__ __align__(16) uint16_t sx[16 * LX], sa1[16 * LH], sa2[16 * LH], sdy[16 * LY], sdz2[16 * LH];
+  __shared__ double part[8];
+  const int kt = blockIdx.x, KT = m.rows / 16;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l = (int)(threadIdx.x & 63);
+  const int c = l & 15, r0 = 4 * (l >> 4);  // column and first row of a result register
+  const int XT = m.inp / 16, YT = m.outp / 16;
+  const int hc = 16 * w + c;  // hidden column of this lane
+  MlpW<4> w1;
+  MlpW<HT> w2, w3[2], w2t;
+  MlpW<12> w3t;
+  w1.load(m.w1, w, XT);
+  w2.load(m.w2, w, HT);
+  const float b1 = m.b1[hc], b2 = m.b2[hc];
+  float b3[2] = {0.0f, 0.0f}, tg[2][4];
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    const int nt = w + 8 * s, j = 16 * nt + c;
+    if (nt >= YT) continue;
+    w3[s].load(m.w3, nt, HT);
+    if (j < m.out) b3[s] = m.b3[j];
+    if (TRAIN) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int b = 16 * kt + r0 + i;
+        const size_t row = m.idx ? m.idx[b] : b;
+        tg[s][i] = j < m.out ? m.t[row * m.out + j] : 0.0f;
+      }
+    }
+  }
+  if (TRAIN) {
+    w3t.load(m.w3t, w, YT);
+    w2t.load(m.w2t, w, HT);
+  }
+  for (int e = threadIdx.x; e < 16 * m.inp; e += 512) {
+    const int r = e / m.inp, j = e % m.inp, b = 16 * kt + r;
+    const size_t row = m.idx ? m.idx[b] : b;
+    sx[r * LX + j] = j < m.in ? mlp_bf16(m.x[row * m.in + j]) : (uint16_t)0;
+  }
+  __syncthreads();
+  if (TRAIN && w < XT) {
+    mlp_bf16x4 f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) f[i] = (short)sx[(r0 + i) * LX + 16 * w + c];
+    m.fx[((size_t)w * KT + kt) * 64 + l] = f;
+  }
+  const size_t frag = ((size_t)w * KT + kt) * 64 + l;
+  float z1[4], z2[4];
+  {
+    const mlp_f32x4 acc = mlp_tile(sx, LX, w1, XT);
+    mlp_bf16x4 f;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int k = k0 + kq + i;
-      a[i] = (short)mlp_bf16(A[(size_t)m * sam + (size_t)k * sak]);
-      b[i] = (short)mlp_bf16(B[(size_t)k * sbk + (size_t)n * sbn]);
+      z1[i] = acc[i] + b1;
+      f[i] = (short)mlp_bf16(mlp_gelu(z1[i]));
+      sa1[(r0 + i) * LH + hc] = (uint16_t)f[i];
     }
-    acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, acc, 0, 0, 0);
+    if (TRAIN) m.fa1[frag] = f;
   }
+  __syncthreads();
+  {
+    const mlp_f32x4 acc = mlp_tile(sa1, LH, w2, HT);
+    mlp_bf16x4 f;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const size_t idx = (size_t)(tm * 16 + kq + i) * ldc + tn * 16 + (l & 15);
-    C[idx] = accumulate ? C[idx] + acc[i] : acc[i];
-  }
-}
-
-// Z[b][j] += bias[j] (j < valid; padding columns zeroed); A = gelu(Z) or Z.
-__global__ void k_mlp_bias_act(int rows, int cols, int valid, float* __restrict__ Z, const float* __restrict__ bias,
-                               float* __restrict__ Aout, int gelu) {
-  const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= (size_t)rows * cols) return;
-  const int j = (int)(idx % cols);
-  const float z = j < valid ? Z[idx] + bias[j] : 0.0f;
-  Z[idx] = z;
-  if (Aout) Aout[idx] = gelu ? (j < valid ? mlp_gelu(z) : 0.0f) : z;
-}
-
-// dY = 2 (Y - T) / (rows * valid) on valid columns; loss partial sums per block.
-__global__ void k_mlp_loss(int rows, int cols, int valid, const float* __restrict__ Y, const float* __restrict__ T,
-                           float* __restrict__ dY, double* __restrict__ loss) {
-  __shared__ double part[256];
-  const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  double e2 = 0.0;
-  if (idx < (size_t)rows * cols) {
-    const int b = (int)(idx / cols), j = (int)(idx % cols);
-    float d = 0.0f;
-    if (j < valid) {
-      const float e = Y[idx] - T[(size_t)b * valid + j];
-      d = 2.0f * e / (float)((double)rows * valid);
-      e2 = (double)e * e;
+    for (int i = 0; i < 4; ++i) {
+      z2[i] = acc[i] + b2;
+      f[i] = (short)mlp_bf16(mlp_gelu(z2[i]));
+      sa2[(r0 + i) * LH + hc] = (uint16_t)f[i];
     }
-    dY[idx] = d;
+    if (TRAIN) m.fa2[frag] = f;
   }
-  part[threadIdx.x] = e2;
   __syncthreads();
-  for (int s = 128; s > 0; s >>= 1) {
-    if ((int)threadIdx.x < s) part[threadIdx.x] += part[threadIdx.x + s];
-    __syncthreads();
+  double e2 = 0.0;
+#pragma unroll
+  for (int s = 0; s < 2; ++s) {
+    const int nt = w + 8 * s;
+    if (nt >= YT) continue;
+    const mlp_f32x4 acc = mlp_tile(sa2, LH, w3[s], HT);
+    const int j = 16 * nt + c;
+    mlp_bf16x4 f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int b = 16 * kt + r0 + i;
+      const float y = j < m.out ? acc[i] + b3[s] : 0.0f;
+      if (!TRAIN) {
+        if (j < m.out) m.y[(size_t)b * m.out + j] = y;
+      } else {
+        float d = 0.0f;
+        if (j < m.out) {
+          const float e = y - tg[s][i];
+          d = 2.0f * e / (float)((double)m.rows * m.out);
+          e2 += (double)e * e;
+        }
+        f[i] = (short)mlp_bf16(d);
+        sdy[(r0 + i) * LY + j] = (uint16_t)f[i];
+        m.dy[(size_t)b * m.outp + j] = d;
+      }
+    }
+    if (TRAIN) m.fdy[((size_t)nt * KT + kt) * 64 + l] = f;
   }
-  if (threadIdx.x == 0) loss[blockIdx.x] = part[0];
+  if (!TRAIN) return;
+  // squared error of the tile, in a fixed order
+#pragma unroll
+  for (int s = 1; s < 64; s <<= 1) e2 += __shfl_xor(e2, s);
+  if (l == 0) part[w] = e2;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double s = 0.0;
+    for (int q = 0; q < 8; ++q) s += part[q];
+    m.loss[kt] = s;
+  }
+  {
+    const mlp_f32x4 acc = mlp_tile(sdy, LY, w3t, YT);
+    mlp_bf16x4 f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float d = acc[i] * mlp_gelu_grad(z2[i]);
+      f[i] = (short)mlp_bf16(d);
+      sdz2[(r0 + i) * LH + hc] = (uint16_t)f[i];
+      m.dz2[(size_t)(16 * kt + r0 + i) * H + hc] = d;
+    }
+    m.fdz2[frag] = f;
+  }
+  __syncthreads();
+  {
+    const mlp_f32x4 acc = mlp_tile(sdz2, LH, w2t, HT);
+    mlp_bf16x4 f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float d = acc[i] * mlp_gelu_grad(z1[i]);
+      f[i] = (short)mlp_bf16(d);
+      m.dz1[(size_t)(16 * kt + r0 + i) * H + hc] = d;
+    }
+    m.fdz1[frag] = f;
+  }
 }
 
-// dZ = dA * gelu'(Z) (in place on dA).
-__global__ void k_mlp_gelu_back(size_t n, float* __restrict__ dA, const float* __restrict__ Z) {
-  const size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx < n) dA[idx] *= mlp_gelu_grad(Z[idx]);
-}
+// Parameters of one Adam step (lr = 0 and adam = 0: gradients only).
+struct MlpStep {
+  float *p, *g, *am, *av;
+  uint16_t *w1, *w2, *w3, *w2t, *w3t;  // operand tiles of the updated weights
+  int off_w1, off_b1, off_w2, off_b2, off_w3, off_b3;
+  int adam;
+  float lr, b1, b2, eps, c1, c2;
+};
 
-// out[j] = sum_b X[b][j] (deterministic: one thread per column).
-// Column sums of a rows x cols row-major matrix (bias gradients): 16 columns
-// per 256-thread block, 16 row phases per column summed through LDS in a fixed
-// order (deterministic).
-__global__ __launch_bounds__(256) void k_mlp_colsum(int rows, int cols, const float* __restrict__ X,
-                                                    float* __restrict__ out) {
+// One parameter's state, loaded before its gradient is known, and its update.
+struct MlpParam {
+  float p, am, av;
+  __device__ __forceinline__ void load(const MlpStep& s, int i) {
+    p = s.p[i];
+    am = s.am[i];
+    av = s.av[i];
+  }
+  __device__ __forceinline__ float update(const MlpStep& s, int i, float gi) {
+    // (fused as written: a training run repeats bit for bit across builds)
+    const float mi = fmaf(1.0f - s.b1, gi, s.b1 * am);
+    const float vi = fmaf(gi, (1.0f - s.b2) * gi, s.b2 * av);
+    s.am[i] = mi;
+    s.av[i] = vi;
+    p -= s.lr * (mi / s.c1) / (sqrtf(vi / s.c2) + s.eps);
+    s.p[i] = p;
+    return p;
+  }
+};
+
+// One wavefront per block.  Blocks 0 .. tiles - 1: a 16x16 tile of a weight
+// gradient, A^T dZ over the batch from the stored fragments (row tiles in
+// ascending order); the rest: 16 bias gradients, the FP32 column sums in 16 row
+// phases joined in a fixed order.  Each then updates its own parameters and
+// their operand tiles, so no gradient goes through memory when training.  Bound
+// by latency like k_mlp_rows (12.2 us with eight fragments in flight and the
+// Adam state loaded after the product, now 5.2 us).
+__global__ __launch_bounds__(64) void k_mlp_weights(MlpBatch m, MlpStep s) {
+  constexpr int H = kMlpHidden, HT = H / 16;
+  const int l = (int)threadIdx.x, KT = m.rows / 16, XT = m.inp / 16, YT = m.outp / 16;
+  int b = blockIdx.x;
+  const int tiles = HT * YT + HT * HT + XT * HT;
+  if (b < tiles) {
+    const mlp_bf16x4 *fa, *fb;
+    uint16_t *wn, *wt = nullptr;
+    int off, N, mts, mt, nt;
+    if (b < HT * YT) {
+      fa = m.fa2, fb = m.fdy, off = s.off_w3, N = m.outp, mts = HT, mt = b / YT, nt = b % YT;
+      wn = s.w3, wt = s.w3t;
+    } else if (b < HT * YT + HT * HT) {
+      b -= HT * YT;
+      fa = m.fa1, fb = m.fdz2, off = s.off_w2, N = H, mts = HT, mt = b / HT, nt = b % HT;
+      wn = s.w2, wt = s.w2t;
+    } else {
+      b -= HT * YT + HT * HT;
+      fa = m.fx, fb = m.fdz1, off = s.off_w1, N = H, mts = XT, mt = b / HT, nt = b % HT;
+      wn = s.w1;
+    }
+    fa += (size_t)mt * KT * 64 + l;
+    fb += (size_t)nt * KT * 64 + l;
+    MlpParam pr[4];
+    const int at0 = off + (16 * mt + 4 * (l >> 4)) * N + 16 * nt + (l & 15);
+    if (s.adam) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) pr[i].load(s, at0 + i * N);
+    }
+    mlp_f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+    constexpr int U = 32;  // row tiles in flight (a batch of 512)
+    for (int k0 = 0; k0 < KT; k0 += U) {
+      mlp_bf16x4 a[U], w[U];
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (k0 + u < KT) {
+          a[u] = fa[(size_t)(k0 + u) * 64];
+          w[u] = fb[(size_t)(k0 + u) * 64];
+        }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (k0 + u < KT) acc = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[u], w[u], acc, 0, 0, 0);
+    }
+    mlp_bf16x4 f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int k = 16 * mt + 4 * (l >> 4) + i, n = 16 * nt + (l & 15);
+      const int at = at0 + i * N;
+      if (!s.adam) {
+        s.g[at] = acc[i];
+        continue;
+      }
+      f[i] = (short)mlp_bf16(pr[i].update(s, at, acc[i]));
+      // W^T[n][k] in its own operand order
+      if (wt)
+        wt[(((size_t)mt * (N / 16) + nt) * 64 + 16 * ((n & 15) >> 2) + (k & 15)) * 4 + (n & 3)] = (uint16_t)f[i];
+    }
+    if (s.adam) reinterpret_cast<mlp_bf16x4*>(wn)[((size_t)nt * mts + mt) * 64 + l] = f;
+    return;
+  }
+  b -= tiles;
+  const float* X;
+  int cols, off;
+  if (b < YT) {
+    X = m.dy, cols = m.outp, off = s.off_b3;
+  } else if (b < YT + HT) {
+    b -= YT;
+    X = m.dz2, cols = H, off = s.off_b2;
+  } else {
+    b -= YT + HT;
+    X = m.dz1, cols = H, off = s.off_b1;
+  }
   __shared__ float part[16][17];
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  const int j = blockIdx.x * 16 + tx;
-  float s = 0.0f;
-  if (j < cols)
-    for (int b = ty; b < rows; b += 16) s += X[(size_t)b * cols + j];
-  part[ty][tx] = s;
+  const int tx = l & 15, tq = 4 * (l >> 4), j = 16 * b + tx;
+  MlpParam pr;
+  if (s.adam) pr.load(s, off + j);
+  float sum[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 16
+  for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+    for (int q = 0; q < 4; ++q) sum[q] += X[(size_t)(16 * kt + tq + q) * cols + j];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) part[tq + q][tx] = sum[q];
   __syncthreads();
-  if (ty == 0 && j < cols) {
+  if (l < 16) {
     float t = 0.0f;
 #pragma unroll
     for (int k = 0; k < 16; ++k) t += part[k][tx];
-    out[j] = t;
+    if (s.adam) pr.update(s, off + j, t);
+    else s.g[off + j] = t;
   }
-}
-
-__global__ void k_mlp_adam(int n, float* __restrict__ p, const float* __restrict__ g, float* __restrict__ m,
-                           float* __restrict__ v, float lr, float b1, float b2, float eps, float c1, float c2) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n) return;
-  const float gi = g[i];
-  const float mi = b1 * m[i] + (1.0f - b1) * gi;
-  const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
-  m[i] = mi;
-  v[i] = vi;
-  p[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
 }
 
 // FP32 K x N row-major -> BF16 in MFMA B-operand tile order (see MlpView).
@@ -138,13 +372,15 @@ __global__ void k_mlp_swizzle(int K, int N, const float* __restrict__ W, uint16_
   out[idx] = mlp_bf16(W[(size_t)k * N + n]);
 }
 
-// Copies sample rows idx[b] of X (n x cols) into a padded batch (rows x ld).
-__global__ void k_mlp_gather(int rows, int cols, int ld, const int* __restrict__ idx, const float* __restrict__ X,
-                             float* __restrict__ out) {
-  const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (size_t)rows * ld) return;
-  const int b = (int)(t / ld), j = (int)(t % ld);
-  out[t] = j < cols ? X[(size_t)idx[b] * cols + j] : 0.0f;
+// The same for the transpose of W: tiles of W^T (N x K).
+__global__ void k_mlp_swizzle_t(int K, int N, const float* __restrict__ W, uint16_t* __restrict__ out) {
+  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
+  if (idx >= K * N) return;
+  const int NT = N / 16;
+  const int i = idx & 3, l = (idx >> 2) & 63, tile = idx >> 8;
+  const int kt = tile % NT, nt = tile / NT;
+  const int n = 16 * kt + 4 * (l >> 4) + i, k = 16 * nt + (l & 15);
+  out[idx] = mlp_bf16(W[(size_t)k * N + n]);
 }
 
 // In-integrator inference path on given states: one wavefront per condition,
@@ -184,12 +420,13 @@ struct Mlp {
   float* sd = nullptr;
   float* zs = nullptr;
   int adam_t = 0;
-  // batch workspace
+  // training's own operand tiles (the integrator keeps reading w1s, w2s, w3s):
+  // one allocation at t1; fresh: they are those of p
+  uint16_t *t1 = nullptr, *t2 = nullptr, *t3 = nullptr, *t2t = nullptr, *t3t = nullptr;
+  bool tiles_fresh = false;
+  // batch workspace (one allocation), for batches of up to cap samples
   int cap = 0;
-  float *X = nullptr, *Z1 = nullptr, *A1 = nullptr, *Z2 = nullptr, *A2 = nullptr, *Y = nullptr, *T = nullptr,
-        *dY = nullptr, *dA2 = nullptr, *dA1 = nullptr;
-  double* loss = nullptr;
-  int* idx = nullptr;
+  char* ws = nullptr;
   std::string err;
 } G;
 
@@ -200,14 +437,8 @@ bool ok(hipError_t e, const char* what) {
 }
 
 void free_ws() {
-  for (float** q : {&G.X, &G.Z1, &G.A1, &G.Z2, &G.A2, &G.Y, &G.T, &G.dY, &G.dA2, &G.dA1}) {
-    if (*q) hipFree(*q);
-    *q = nullptr;
-  }
-  if (G.loss) hipFree(G.loss);
-  if (G.idx) hipFree(G.idx);
-  G.loss = nullptr;
-  G.idx = nullptr;
+  if (G.ws) hipFree(G.ws);
+  G.ws = nullptr;
   G.cap = 0;
 }
 
@@ -222,87 +453,118 @@ void free_all() {
     if (*q) hipFree(*q);
     *q = nullptr;
   }
-  for (uint16_t** q : {&G.w1s, &G.w2s, &G.w3s}) {
+  for (uint16_t** q : {&G.w1s, &G.w2s, &G.w3s, &G.t1}) {
     if (*q) hipFree(*q);
     *q = nullptr;
   }
   G.n = 0;
 }
 
+int blocks_for(size_t n, int t = 256) { return (int)((n + t - 1) / t); }
+
+// The batch's buffers in the workspace (base 0: their total size in `bytes`).
+MlpBatch batch_buffers(int B, char* base, size_t* bytes) {
+  const size_t H = kMlpHidden;
+  size_t at = 0;
+  auto take = [&](size_t n) {
+    char* p = base + at;
+    at += (n + 255) / 256 * 256;
+    return p;
+  };
+  MlpBatch m{};
+  m.in = G.in;
+  m.inp = G.inp;
+  m.out = G.out;
+  m.outp = G.outp;
+  m.rows = B;
+  m.w1 = G.t1;
+  m.w2 = G.t2;
+  m.w3 = G.t3;
+  m.w2t = G.t2t;
+  m.w3t = G.t3t;
+  m.b1 = G.p + G.off_b1;
+  m.b2 = G.p + G.off_b2;
+  m.b3 = G.p + G.off_b3;
+  m.fx = (mlp_bf16x4*)take((size_t)B * G.inp * 2);
+  m.fa1 = (mlp_bf16x4*)take((size_t)B * H * 2);
+  m.fa2 = (mlp_bf16x4*)take((size_t)B * H * 2);
+  m.fdy = (mlp_bf16x4*)take((size_t)B * G.outp * 2);
+  m.fdz2 = (mlp_bf16x4*)take((size_t)B * H * 2);
+  m.fdz1 = (mlp_bf16x4*)take((size_t)B * H * 2);
+  m.dy = (float*)take((size_t)B * G.outp * 4);
+  m.dz2 = (float*)take((size_t)B * H * 4);
+  m.dz1 = (float*)take((size_t)B * H * 4);
+  // host-array calls: the uploaded samples and targets, the outputs
+  m.x = (float*)take((size_t)B * G.in * 4);
+  m.t = (float*)take((size_t)B * G.out * 4);
+  m.y = (float*)take((size_t)B * G.out * 4);
+  m.loss = (double*)take((size_t)(B / 16) * sizeof(double));
+  *bytes = at;
+  return m;
+}
+
 bool ensure_ws(int B) {
   if (B <= G.cap) return true;
   free_ws();
-  const size_t H = kMlpHidden;
-  bool good = ok(hipMalloc(&G.X, (size_t)B * G.inp * 4), "hipMalloc") &&
-              ok(hipMalloc(&G.Z1, (size_t)B * H * 4), "hipMalloc") && ok(hipMalloc(&G.A1, (size_t)B * H * 4), "hipMalloc") &&
-              ok(hipMalloc(&G.Z2, (size_t)B * H * 4), "hipMalloc") && ok(hipMalloc(&G.A2, (size_t)B * H * 4), "hipMalloc") &&
-              ok(hipMalloc(&G.Y, (size_t)B * G.outp * 4), "hipMalloc") &&
-              ok(hipMalloc(&G.T, (size_t)B * G.out * 4), "hipMalloc") &&
-              ok(hipMalloc(&G.dY, (size_t)B * G.outp * 4), "hipMalloc") &&
-              ok(hipMalloc(&G.dA2, (size_t)B * H * 4), "hipMalloc") && ok(hipMalloc(&G.dA1, (size_t)B * H * 4), "hipMalloc") &&
-              ok(hipMalloc(&G.loss, (size_t)((B * G.outp + 255) / 256) * sizeof(double)), "hipMalloc") &&
-              ok(hipMalloc(&G.idx, (size_t)B * sizeof(int)), "hipMalloc");
-  if (!good) {
-    free_ws();
-    return false;
-  }
+  size_t bytes = 0;
+  batch_buffers(B, nullptr, &bytes);
+  if (!ok(hipMalloc(&G.ws, bytes), "hipMalloc")) return false;
   G.cap = B;
   return true;
 }
-
-int blocks_for(size_t n, int t = 256) { return (int)((n + t - 1) / t); }
-
-void gemm(int M, int N, int K, const float* A, int sam, int sak, const float* B, int sbk, int sbn, float* C,
-          int ldc, int accumulate) {
-  const int tiles = (M / 16) * (N / 16);
-  hipLaunchKernelGGL(k_mlp_gemm, dim3((tiles + 3) / 4), dim3(256), 0, 0, M, N, K, A, sam, sak, B, sbk, sbn, C,
-                     ldc, accumulate);
+MlpBatch workspace_batch(int B) {
+  size_t bytes = 0;
+  return batch_buffers(B, G.ws, &bytes);
 }
 
-// Forward pass of a prepared batch in G.X (B x inp); outputs in G.Y (B x outp).
-void forward(int B) {
-  const int H = kMlpHidden;
-  float *W1 = G.p + G.off_w1, *b1 = G.p + G.off_b1, *W2 = G.p + G.off_w2, *b2 = G.p + G.off_b2,
-        *W3 = G.p + G.off_w3, *b3 = G.p + G.off_b3;
-  gemm(B, H, G.inp, G.X, G.inp, 1, W1, H, 1, G.Z1, H, 0);
-  hipLaunchKernelGGL(k_mlp_bias_act, dim3(blocks_for((size_t)B * H)), dim3(256), 0, 0, B, H, H, G.Z1, b1, G.A1, 1);
-  gemm(B, H, H, G.A1, H, 1, W2, H, 1, G.Z2, H, 0);
-  hipLaunchKernelGGL(k_mlp_bias_act, dim3(blocks_for((size_t)B * H)), dim3(256), 0, 0, B, H, H, G.Z2, b2, G.A2, 1);
-  gemm(B, G.outp, H, G.A2, H, 1, W3, G.outp, 1, G.Y, G.outp, 0);
-  hipLaunchKernelGGL(k_mlp_bias_act, dim3(blocks_for((size_t)B * G.outp)), dim3(256), 0, 0, B, G.outp, G.out, G.Y,
-                     b3, (float*)nullptr, 0);
+MlpStep step_params(int adam, float lr, float c1, float c2) {
+  MlpStep s{};
+  s.p = G.p;
+  s.g = G.g;
+  s.am = G.am;
+  s.av = G.av;
+  s.w1 = G.t1;
+  s.w2 = G.t2;
+  s.w3 = G.t3;
+  s.w2t = G.t2t;
+  s.w3t = G.t3t;
+  s.off_w1 = G.off_w1;
+  s.off_b1 = G.off_b1;
+  s.off_w2 = G.off_w2;
+  s.off_b2 = G.off_b2;
+  s.off_w3 = G.off_w3;
+  s.off_b3 = G.off_b3;
+  s.adam = adam;
+  s.lr = lr;
+  s.b1 = 0.9f;
+  s.b2 = 0.999f;
+  s.eps = 1e-8f;
+  s.c1 = c1;
+  s.c2 = c2;
+  return s;
 }
 
-// Loss and gradients (into G.g) of the batch in G.X / G.T; returns the summed
-// squared error.
-bool loss_grad(int B, double* sse) {
+// Squared error and gradients of a batch; with an Adam step, the parameters'
+// update in place of the gradients.
+void launch_batch(const MlpBatch& m, const MlpStep& s) {
+  const int HT = kMlpHidden / 16, XT = m.inp / 16, YT = m.outp / 16;
+  hipLaunchKernelGGL(k_mlp_rows<true>, dim3(m.rows / 16), dim3(512), 0, 0, m);
+  hipLaunchKernelGGL(k_mlp_weights, dim3(HT * YT + HT * HT + XT * HT + YT + 2 * HT), dim3(64), 0, 0, m, s);
+}
+
+// Training's operand tiles from the FP32 parameters (an Adam step keeps them).
+bool refresh_training_tiles() {
+  if (G.tiles_fresh) return true;
   const int H = kMlpHidden;
-  forward(B);
-  const int nb = blocks_for((size_t)B * G.outp);
-  hipLaunchKernelGGL(k_mlp_loss, dim3(nb), dim3(256), 0, 0, B, G.outp, G.out, G.Y, G.T, G.dY, G.loss);
-  float *W2 = G.p + G.off_w2, *W3 = G.p + G.off_w3;
-  float *gW1 = G.g + G.off_w1, *gb1 = G.g + G.off_b1, *gW2 = G.g + G.off_w2, *gb2 = G.g + G.off_b2,
-        *gW3 = G.g + G.off_w3, *gb3 = G.g + G.off_b3;
-  // layer 3
-  gemm(H, G.outp, B, G.A2, 1, H, G.dY, G.outp, 1, gW3, G.outp, 0);
-  hipLaunchKernelGGL(k_mlp_colsum, dim3((G.outp + 15) / 16), dim3(256), 0, 0, B, G.outp, G.dY, gb3);
-  gemm(B, H, G.outp, G.dY, G.outp, 1, W3, 1, G.outp, G.dA2, H, 0);
-  hipLaunchKernelGGL(k_mlp_gelu_back, dim3(blocks_for((size_t)B * H)), dim3(256), 0, 0, (size_t)B * H, G.dA2, G.Z2);
-  // layer 2
-  gemm(H, H, B, G.A1, 1, H, G.dA2, H, 1, gW2, H, 0);
-  hipLaunchKernelGGL(k_mlp_colsum, dim3((H + 15) / 16), dim3(256), 0, 0, B, H, G.dA2, gb2);
-  gemm(B, H, H, G.dA2, H, 1, W2, 1, H, G.dA1, H, 0);
-  hipLaunchKernelGGL(k_mlp_gelu_back, dim3(blocks_for((size_t)B * H)), dim3(256), 0, 0, (size_t)B * H, G.dA1, G.Z1);
-  // layer 1
-  gemm(G.inp, H, B, G.X, 1, G.inp, G.dA1, H, 1, gW1, H, 0);
-  hipLaunchKernelGGL(k_mlp_colsum, dim3((H + 15) / 16), dim3(256), 0, 0, B, H, G.dA1, gb1);
-  if (!ok(hipGetLastError(), "mlp backward")) return false;
-  std::vector<double> part(nb);
-  if (!ok(hipMemcpy(part.data(), G.loss, nb * sizeof(double), hipMemcpyDeviceToHost), "hipMemcpy")) return false;
-  double s = 0.0;
-  for (double v : part) s += v;
-  *sse = s;
-  return true;
+  hipLaunchKernelGGL(k_mlp_swizzle, dim3(blocks_for((size_t)G.inp * H)), dim3(256), 0, 0, G.inp, H, G.p + G.off_w1, G.t1);
+  hipLaunchKernelGGL(k_mlp_swizzle, dim3(blocks_for((size_t)H * H)), dim3(256), 0, 0, H, H, G.p + G.off_w2, G.t2);
+  hipLaunchKernelGGL(k_mlp_swizzle, dim3(blocks_for((size_t)H * G.outp)), dim3(256), 0, 0, H, G.outp, G.p + G.off_w3,
+                     G.t3);
+  hipLaunchKernelGGL(k_mlp_swizzle_t, dim3(blocks_for((size_t)H * H)), dim3(256), 0, 0, H, H, G.p + G.off_w2, G.t2t);
+  hipLaunchKernelGGL(k_mlp_swizzle_t, dim3(blocks_for((size_t)H * G.outp)), dim3(256), 0, 0, H, G.outp,
+                     G.p + G.off_w3, G.t3t);
+  G.tiles_fresh = ok(hipGetLastError(), "mlp swizzle");
+  return G.tiles_fresh;
 }
 
 bool refresh_swizzled() {
@@ -313,16 +575,6 @@ bool refresh_swizzled() {
   hipLaunchKernelGGL(k_mlp_swizzle, dim3(blocks_for((size_t)H * G.outp)), dim3(256), 0, 0, H, G.outp,
                      G.p + G.off_w3, G.w3s);
   return ok(hipGetLastError(), "mlp swizzle") && ok(hipDeviceSynchronize(), "mlp swizzle");
-}
-
-// Uploads a host batch (x: B x in, t: B x out, normalized) into the padded workspace.
-bool upload_batch(int B, const float* x, const float* t) {
-  std::vector<float> xp((size_t)B * G.inp, 0.0f);
-  for (int b = 0; b < B; ++b)
-    for (int j = 0; j < G.in; ++j) xp[(size_t)b * G.inp + j] = x[(size_t)b * G.in + j];
-  if (!ok(hipMemcpy(G.X, xp.data(), xp.size() * 4, hipMemcpyHostToDevice), "hipMemcpy")) return false;
-  if (t && !ok(hipMemcpy(G.T, t, (size_t)B * G.out * 4, hipMemcpyHostToDevice), "hipMemcpy")) return false;
-  return true;
 }
 
 }  // namespace
@@ -389,6 +641,7 @@ int accelerInt_mlp_init(int n_states, unsigned seed) {
               ok(hipMalloc(&G.w1s, (size_t)G.inp * H * 2), "hipMalloc") &&
               ok(hipMalloc(&G.w2s, (size_t)H * H * 2), "hipMalloc") &&
               ok(hipMalloc(&G.w3s, (size_t)H * G.outp * 2), "hipMalloc") &&
+              ok(hipMalloc(&G.t1, ((size_t)G.inp * H + 2 * (size_t)H * H + 2 * (size_t)H * G.outp) * 2), "hipMalloc") &&
               ok(hipMalloc(&G.mu, G.inp * 4), "hipMalloc") && ok(hipMalloc(&G.sd, G.inp * 4), "hipMalloc") &&
               ok(hipMalloc(&G.zs, G.outp * 4), "hipMalloc") &&
               ok(hipMemcpy(G.p, p.data(), G.count * 4, hipMemcpyHostToDevice), "hipMemcpy") &&
@@ -401,6 +654,11 @@ int accelerInt_mlp_init(int n_states, unsigned seed) {
     free_all();
     return -1;
   }
+  G.t2 = G.t1 + (size_t)G.inp * H;
+  G.t2t = G.t2 + (size_t)H * H;
+  G.t3 = G.t2t + (size_t)H * H;
+  G.t3t = G.t3 + (size_t)H * G.outp;
+  G.tiles_fresh = false;
   G.adam_t = 0;
   return 0;
 }
@@ -420,6 +678,7 @@ int accelerInt_mlp_set_params(const float* in, int count) {
     G.err = "accelerInt_mlp_set_params: no network or wrong count";
     return -1;
   }
+  G.tiles_fresh = false;
   if (!ok(hipMemcpy(G.p, in, (size_t)count * 4, hipMemcpyHostToDevice), "hipMemcpy")) return -1;
   return refresh_swizzled() ? 0 : -1;
 }
@@ -451,9 +710,18 @@ int accelerInt_mlp_loss_grad(int B, const float* x, const float* t, float* grad,
     G.err = "accelerInt_mlp_loss_grad: no network, or B not a positive multiple of 16";
     return -1;
   }
-  if (!ensure_ws(B) || !upload_batch(B, x, t)) return -1;
+  if (!ensure_ws(B)) return -1;
+  const MlpBatch m = workspace_batch(B);
+  if (!ok(hipMemcpy((void*)m.x, x, (size_t)B * G.in * 4, hipMemcpyHostToDevice), "hipMemcpy") ||
+      !ok(hipMemcpy((void*)m.t, t, (size_t)B * G.out * 4, hipMemcpyHostToDevice), "hipMemcpy") ||
+      !refresh_training_tiles())
+    return -1;
+  launch_batch(m, step_params(0, 0.0f, 1.0f, 1.0f));
+  if (!ok(hipGetLastError(), "mlp backward")) return -1;
+  std::vector<double> part(B / 16);
+  if (!ok(hipMemcpy(part.data(), m.loss, part.size() * sizeof(double), hipMemcpyDeviceToHost), "hipMemcpy")) return -1;
   double sse = 0.0;
-  if (!loss_grad(B, &sse)) return -1;
+  for (double v : part) sse += v;
   if (loss) *loss = (float)(sse / ((double)B * G.out));
   return ok(hipMemcpy(grad, G.g, (size_t)G.count * 4, hipMemcpyDeviceToHost), "hipMemcpy") ? 0 : -1;
 }
@@ -463,15 +731,21 @@ int accelerInt_mlp_predict(int B, const float* x, float* y) {
     G.err = "accelerInt_mlp_predict: no network, or B not a positive multiple of 16";
     return -1;
   }
-  if (!ensure_ws(B) || !upload_batch(B, x, nullptr)) return -1;
-  forward(B);
-  std::vector<float> yp((size_t)B * G.outp);
-  if (!ok(hipMemcpy(yp.data(), G.Y, yp.size() * 4, hipMemcpyDeviceToHost), "hipMemcpy")) return -1;
-  for (int b = 0; b < B; ++b)
-    for (int j = 0; j < G.out; ++j) y[(size_t)b * G.out + j] = yp[(size_t)b * G.outp + j];
-  return 0;
+  if (!ensure_ws(B)) return -1;
+  const MlpBatch m = workspace_batch(B);
+  if (!ok(hipMemcpy((void*)m.x, x, (size_t)B * G.in * 4, hipMemcpyHostToDevice), "hipMemcpy") ||
+      !refresh_training_tiles())
+    return -1;
+  hipLaunchKernelGGL(k_mlp_rows<false>, dim3(B / 16), dim3(512), 0, 0, m);
+  return ok(hipGetLastError(), "mlp forward") &&
+                 ok(hipMemcpy(y, m.y, (size_t)B * G.out * 4, hipMemcpyDeviceToHost), "hipMemcpy")
+             ? 0
+             : -1;
 }
 
+// Adam over shuffled batches.  An epoch's batches are launched without waiting
+// for any of them; the next epoch's permutation is drawn while they run, and the
+// epoch's squared errors come back in one copy at its end.
 int accelerInt_mlp_train(int n, const float* x_dev, const float* t_dev, int epochs, int batch, float lr,
                          unsigned seed, float* loss_per_epoch) {
   if (!G.n || n < batch || batch <= 0 || batch % 16 || epochs <= 0 || !x_dev || !t_dev) {
@@ -482,42 +756,49 @@ int accelerInt_mlp_train(int n, const float* x_dev, const float* t_dev, int epoc
   std::mt19937 rng(seed);
   std::vector<int> perm(n);
   for (int i = 0; i < n; ++i) perm[i] = i;
+  const int steps = n / batch, tiles = batch / 16;
+  std::vector<double> part((size_t)steps * tiles);
   int* d_perm = nullptr;
-  if (!ok(hipMalloc(&d_perm, (size_t)n * sizeof(int)), "hipMalloc")) return -1;
-  const int steps = n / batch;
-  int rc = 0;
+  double* d_loss = nullptr;
+  int rc = -1;
+  if (ok(hipMalloc(&d_perm, (size_t)n * sizeof(int)), "hipMalloc") &&
+      ok(hipMalloc(&d_loss, part.size() * sizeof(double)), "hipMalloc") && refresh_training_tiles())
+    rc = 0;
+  MlpBatch m = workspace_batch(batch);
+  m.x = x_dev;
+  m.t = t_dev;
+  if (rc == 0) std::shuffle(perm.begin(), perm.end(), rng);
   for (int ep = 0; ep < epochs && rc == 0; ++ep) {
-    std::shuffle(perm.begin(), perm.end(), rng);
     if (!ok(hipMemcpy(d_perm, perm.data(), (size_t)n * sizeof(int), hipMemcpyHostToDevice), "hipMemcpy")) {
       rc = -1;
       break;
     }
-    double sse = 0.0;
     for (int s = 0; s < steps; ++s) {
-      const int* ib = d_perm + (size_t)s * batch;
-      hipLaunchKernelGGL(k_mlp_gather, dim3(blocks_for((size_t)batch * G.inp)), dim3(256), 0, 0, batch, G.in,
-                         G.inp, ib, x_dev, G.X);
-      hipLaunchKernelGGL(k_mlp_gather, dim3(blocks_for((size_t)batch * G.out)), dim3(256), 0, 0, batch, G.out,
-                         G.out, ib, t_dev, G.T);
-      double part = 0.0;
-      if (!loss_grad(batch, &part)) {
-        rc = -1;
-        break;
-      }
-      sse += part;
+      m.idx = d_perm + (size_t)s * batch;
+      m.loss = d_loss + (size_t)s * tiles;
       ++G.adam_t;
-      const float b1 = 0.9f, b2 = 0.999f;
-      const float c1 = 1.0f - powf(b1, (float)G.adam_t), c2 = 1.0f - powf(b2, (float)G.adam_t);
-      hipLaunchKernelGGL(k_mlp_adam, dim3(blocks_for(G.count)), dim3(256), 0, 0, G.count, G.p, G.g, G.am, G.av, lr,
-                         b1, b2, 1e-8f, c1, c2);
+      const float c1 = 1.0f - powf(0.9f, (float)G.adam_t), c2 = 1.0f - powf(0.999f, (float)G.adam_t);
+      launch_batch(m, step_params(1, lr, c1, c2));
     }
+    if (!ok(hipGetLastError(), "mlp training")) {
+      rc = -1;
+      break;
+    }
+    if (ep + 1 < epochs) std::shuffle(perm.begin(), perm.end(), rng);
+    if (!ok(hipMemcpy(part.data(), d_loss, part.size() * sizeof(double), hipMemcpyDeviceToHost), "hipMemcpy")) {
+      rc = -1;
+      break;
+    }
+    double sse = 0.0;
+    for (double v : part) sse += v;
     if (loss_per_epoch) loss_per_epoch[ep] = (float)(sse / ((double)steps * batch * G.out));
-    if (rc == 0 && !std::isfinite(sse)) {
+    if (!std::isfinite(sse)) {
       G.err = "accelerInt_mlp_train: non-finite loss (training diverged or non-finite samples)";
       rc = -1;
     }
   }
-  hipFree(d_perm);
+  if (d_perm) hipFree(d_perm);
+  if (d_loss) hipFree(d_loss);
   if (rc == 0 && !refresh_swizzled()) rc = -1;
   return rc;
 }
