@@ -250,7 +250,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(WPE, WPE)
   // out of the vector register file
   const int g = G == 64 ? __builtin_amdgcn_readfirstlane(threadIdx.x / G) : (int)(threadIdx.x / G);
   Mech::block_init(mp, lds_dyn);
-  typename Mech::Ctx ctx(mp, g, lds_dyn, Radau<Mech, G, R, MT>::kNeedsScratch);
+  typename Mech::Ctx ctx(mp, g, lds_dyn);
   // learned start: the group's predicted stages after the mechanism's LDS
   double* zs = LS ? lds_dyn + start_off + (size_t)g * 3 * G * R : nullptr;
   char* gws = group_ws(P, (size_t)blockIdx.x * (BLOCK / G) + g);
@@ -275,19 +275,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 1))) voi
   double* region = lds_dyn + off_regions + (size_t)w * region_doubles;
   if (q112.num > 0) {
     // a wave per 112-state condition; its tables stay in global memory (L2)
-    MechKinetics112::Ctx ctx(mp112, mp112.blob, region, false);
+    MechKinetics112::Ctx ctx(mp112, mp112.blob, region);
     run_queue<MechKinetics112, 64, 2, MT>(q112, t_start, t_end, step, P, ctx, nullptr,
                                           group_ws(P, (size_t)blockIdx.x * 4 + w));
   }
   {
-    MechKinetics54::Ctx ctx(mp54, lds_dyn, region, false);
+    MechKinetics54::Ctx ctx(mp54, lds_dyn, region);
     run_queue<MechKinetics54, 64, 1, MT>(q54, t_start, t_end, step, P, ctx);
   }
   {
-    constexpr bool scratch = Radau<MechKinetics14, 16, 1, MT>::kNeedsScratch;
     const int g = (threadIdx.x & 63) / 16;
-    MechKinetics14::Ctx ctx(mp14, lds_dyn + off14, region + (size_t)g * MechKinetics14::group_doubles(mp14.nr, scratch),
-                            scratch);
+    MechKinetics14::Ctx ctx(mp14, lds_dyn + off14, region + (size_t)g * MechKinetics14::group_doubles(mp14.nr));
     run_queue<MechKinetics14, 16, 1, MT>(q14, t_start, t_end, step, P, ctx);
   }
 }
@@ -327,7 +325,7 @@ __global__ __launch_bounds__(BLOCK) void k_eval_callbacks(int num, double t,
     const int r = ln + G * q;
     yl[q] = (r < N) ? y[(size_t)c * N + r] : 0.0;
   }
-  typename Mech::Ctx ctx(mp, g, lds_dyn, false);
+  typename Mech::Ctx ctx(mp, g, lds_dyn);
   if constexpr (MechGlobal<Mech>::value > 0)  // a workspace slice per condition
     ctx.bind_global(reinterpret_cast<double*>(gws) + (size_t)c * MechGlobal<Mech>::value);
   Mech::template dydt<G, R>(ctx, t, pr[c], yl, f);
@@ -368,7 +366,7 @@ hipError_t launch_eval(int num, double t, const double* pr, const double* y, dou
   const int blocks = (num + GPB - 1) / GPB;
   if (blocks == 0) return hipSuccess;
   auto kern = k_eval_callbacks<Mech, G, R, BLOCK>;
-  const size_t lds = Mech::lds_bytes(mp, GPB, false);
+  const size_t lds = Mech::lds_bytes(mp, GPB);
   hipError_t e = allow_lds(kern, lds);
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL(kern, dim3(blocks), dim3(BLOCK), lds, s, num, t, pr, y, dy, jac, mp, gws);
@@ -404,7 +402,7 @@ hipError_t launch_radau(int num, double t_start, double t_end, double step, cons
                         const typename Mech::Params& mp, hipStream_t s, float* cost = nullptr) {
   constexpr int GPB = BLOCK / G;
   auto kern = k_radau<Mech, G, R, BLOCK, WPE, MT, LS>;
-  const size_t lds_mech = Mech::lds_bytes(mp, GPB, Radau<Mech, G, R, MT>::kNeedsScratch);
+  const size_t lds_mech = Mech::lds_bytes(mp, GPB);
   // learned start: 3 stages x R rows x G lanes of doubles per group after the mechanism's share
   const size_t lds = lds_mech + (LS ? (size_t)GPB * 3 * G * R * sizeof(double) : 0);
   static int resident = 0;     // blocks per device that fit at once, per instantiation
@@ -922,13 +920,12 @@ hipError_t launch_hetero(int n112, const double* pr112, double* y112, int* codes
                          double* y54, int* codes54, int n14, const double* pr14, double* y14, int* codes14,
                          double t_start, double t_end, double step, const SolverParams& P, hipStream_t s) {
   constexpr bool kMixed = std::is_same<MT, float>::value;
-  constexpr bool sc14 = Radau<MechKinetics14, 16, 1, MT>::kNeedsScratch;
   auto kern = k_radau_hetero<MT>;
   const int off14 = S.kp54.lds_bytes / 8;
   const int off_regions = off14 + S.kp14.lds_bytes / 8;
-  const size_t r54 = MechKinetics54::group_doubles(S.kp54.nr, false);
-  const size_t r14 = 4 * MechKinetics14::group_doubles(S.kp14.nr, sc14);
-  const size_t r112 = n112 > 0 ? MechKinetics112::group_doubles(S.kp112.nr, false) : 0;
+  const size_t r54 = MechKinetics54::group_doubles(S.kp54.nr);
+  const size_t r14 = 4 * MechKinetics14::group_doubles(S.kp14.nr);
+  const size_t r112 = n112 > 0 ? MechKinetics112::group_doubles(S.kp112.nr) : 0;
   size_t region_sz = r54 > r14 ? r54 : r14;
   region_sz = region_sz > r112 ? region_sz : r112;
   const int region = (int)region_sz;

@@ -1,7 +1,7 @@
 // Device LU without integration: the LU routines the integrator runs at each
 // order and precision (radau_core.hpp: the row LU lu_real / lu_cplx with
-// implicit interchanges; at order 14 in FP64 the column LU clu_real /
-// clu_cplx with explicit ones) on caller matrices, so that their pivot
+// implicit interchanges; at order 14 row16_lu_real / row16_lu_cplx, which leave
+// the rows in LAPACK's order) on caller matrices, so that their pivot
 // choice, factors and zero-pivot report can be checked one to one against
 // LAPACK dgetrf_/zgetrf_, the routines the reference calls in RK_Decomp
 // (radau2a.c:273,277); optionally also the matching triangular solves on one
@@ -89,59 +89,49 @@ __global__ __launch_bounds__(64) void k_factor_test(int num, const double* __res
   }
 }
 
-// Order 14 in FP64: the column LU (lane j holds column j, rows physically
-// interchanged; rmap byte k = the original row now at position k, which is
-// also the row chosen at step k), then the factors turned into rows through
-// LDS for the row-layout solves, as the integrator does.
-template <bool CPLX>
-__global__ __launch_bounds__(64) void k_factor_test_col(int num, const double* __restrict__ a_re,
-                                                        const double* __restrict__ a_im,
-                                                        const double* __restrict__ b_re,
-                                                        const double* __restrict__ b_im, double* __restrict__ lu_re,
-                                                        double* __restrict__ lu_im, int* __restrict__ perm_out,
-                                                        int* __restrict__ info_out, double* __restrict__ x_re,
-                                                        double* __restrict__ x_im) {
+// Order 14: the LU of 16-lane groups, rows moved to the lanes of their LAPACK
+// positions (src = the original row now in this lane, which is also the row
+// chosen at that step), and its solves.
+template <class T, bool CPLX>
+__global__ __launch_bounds__(64) void k_factor_test_16(int num, const double* __restrict__ a_re,
+                                                       const double* __restrict__ a_im,
+                                                       const double* __restrict__ b_re,
+                                                       const double* __restrict__ b_im, double* __restrict__ lu_re,
+                                                       double* __restrict__ lu_im, int* __restrict__ perm_out,
+                                                       int* __restrict__ info_out, double* __restrict__ x_re,
+                                                       double* __restrict__ x_im) {
   constexpr int N = 14, G = 16;
-  __shared__ double scratch[64 / G][N * N];
   const int ln = Grp<G>::lane();
-  const int g = (int)threadIdx.x / G;
-  const int c = blockIdx.x * (64 / G) + g;
+  const int c = blockIdx.x * (64 / G) + (int)threadIdx.x / G;
   if (c >= num) return;  // whole groups leave together
   const size_t base = (size_t)c * N * N;
-  double ar[N], ai[N];
+  T ar[N], ai[N];
 #pragma unroll
-  for (int i = 0; i < N; ++i) {
-    ar[i] = ln < N ? a_re[base + (size_t)i * N + ln] : 0.0;
-    ai[i] = (CPLX && ln < N) ? a_im[base + (size_t)i * N + ln] : 0.0;
+  for (int j = 0; j < N; ++j) {
+    ar[j] = ln < N ? (T)a_re[base + (size_t)ln * N + j] : T(0);
+    ai[j] = (CPLX && ln < N) ? (T)a_im[base + (size_t)ln * N + j] : T(0);
   }
-  RowMap<N> rmap;
-  double rdr = 0.0, rdi = 0.0;
-  int info = 0;
-  if constexpr (CPLX) clu_cplx<N, G>(ar, ai, rmap, rdr, rdi, info);
-  else clu_real<N, G>(ar, rmap, rdr, info);
+  int src = 0, info = 0;
+  T rdr, rdi = T(0);
+  if constexpr (CPLX) row16_lu_cplx<N, T>(ar, ai, src, rdr, rdi, info);
+  else row16_lu_real<N, T>(ar, src, rdr, info);
   if (ln < N) {
 #pragma unroll
-    for (int i = 0; i < N; ++i) {
-      lu_re[base + (size_t)i * N + ln] = ar[i];
-      if (CPLX) lu_im[base + (size_t)i * N + ln] = ai[i];
+    for (int j = 0; j < N; ++j) {
+      lu_re[base + (size_t)ln * N + j] = (double)ar[j];
+      if (CPLX) lu_im[base + (size_t)ln * N + j] = (double)ai[j];
     }
+    perm_out[(size_t)c * N + ln] = src;
   }
-  if (ln == 0) {
-    for (int k = 0; k < N; ++k) perm_out[(size_t)c * N + k] = rmap.get(k);
-    info_out[c] = info;
-  }
+  if (ln == 0) info_out[c] = info;
   if (b_re) {  // uniform over the launch
-    double rr[N], ri[N];
-    transpose_cols_to_rows<N, G>(ar, rr, scratch[g]);
-    if (CPLX) transpose_cols_to_rows<N, G>(ai, ri, scratch[g]);
-    const int src = rmap.get(ln);
-    double br = ln < N ? b_re[(size_t)c * N + ln] : 0.0;
-    double bi = (CPLX && ln < N) ? b_im[(size_t)c * N + ln] : 0.0;
-    if constexpr (CPLX) rsolve_cplx<N, G>(rr, ri, src, rdr, rdi, br, bi);
-    else rsolve_real<N, G>(rr, src, rdr, br);
+    T br = ln < N ? (T)b_re[(size_t)c * N + ln] : T(0);
+    T bi = (CPLX && ln < N) ? (T)b_im[(size_t)c * N + ln] : T(0);
+    if constexpr (CPLX) rsolve_cplx<N, G, T>(ar, ai, src, rdr, rdi, br, bi);
+    else rsolve_real<N, G, T>(ar, src, rdr, br);
     if (ln < N) {
-      x_re[(size_t)c * N + ln] = br;
-      if (CPLX) x_im[(size_t)c * N + ln] = bi;
+      x_re[(size_t)c * N + ln] = (double)br;
+      if (CPLX) x_im[(size_t)c * N + ln] = (double)bi;
     }
   }
 }
@@ -279,19 +269,18 @@ hipError_t launch_factor_test(int n, bool fp32, bool cplx, int num, const double
   }
   switch (n) {
     case 2: return launch_order<2, 1, 2>(fp32, cplx, num, are, aim, bre, bim, lre, lim, perm, info, xre, xim, s);
-    case 14:
-      if (!fp32) {
-        const int blocks = (num + 3) / 4;
-        if (cplx)
-          hipLaunchKernelGGL(k_factor_test_col<true>, dim3(blocks), dim3(64), 0, s, num, are, aim, bre, bim, lre, lim,
-                             perm, info, xre, xim);
-        else
-          hipLaunchKernelGGL(k_factor_test_col<false>, dim3(blocks), dim3(64), 0, s, num, are, aim, bre, bim, lre,
-                             lim, perm, info, xre, xim);
-        return hipGetLastError();
-      }
-      return cplx ? launch_one<14, 16, 1, float, true>(num, are, aim, bre, bim, lre, lim, perm, info, xre, xim, s)
-                  : launch_one<14, 16, 1, float, false>(num, are, aim, bre, bim, lre, lim, perm, info, xre, xim, s);
+    case 14: {
+      const dim3 blocks((num + 3) / 4);
+#define LAUNCH_16(T, CPLX)                                                                                       \
+  hipLaunchKernelGGL((k_factor_test_16<T, CPLX>), blocks, dim3(64), 0, s, num, are, aim, bre, bim, lre, lim, perm, \
+                     info, xre, xim)
+      if (fp32 && cplx) LAUNCH_16(float, true);
+      else if (fp32) LAUNCH_16(float, false);
+      else if (cplx) LAUNCH_16(double, true);
+      else LAUNCH_16(double, false);
+#undef LAUNCH_16
+      return hipGetLastError();
+    }
     case 54: return launch_order<54, 64, 1>(fp32, cplx, num, are, aim, bre, bim, lre, lim, perm, info, xre, xim, s);
     default: return hipErrorInvalidValue;
   }

@@ -58,17 +58,17 @@ struct MechFD {
     double atol, rtol;
     int order;  // 1, 2, 4 or 6
   };
-  static size_t lds_bytes(const Params& p, int groups, bool scratch) {
-    return Base::lds_bytes(p.base, groups, scratch);
+  static size_t lds_bytes(const Params& p, int groups) {
+    return Base::lds_bytes(p.base, groups);
   }
   __device__ __forceinline__ static void block_init(const Params& p, double* lds) { Base::block_init(p.base, lds); }
   struct Ctx : Base::Ctx {
     double atol, rtol;
     int order;
-    __device__ Ctx(const Params& p, int g, double* lds, bool scratch)
-        : Base::Ctx(p.base, g, lds, scratch), atol(p.atol), rtol(p.rtol), order(p.order) {}
-    __device__ Ctx(const Params& p, const double* tables, double* group, bool scratch)
-        : Base::Ctx(p.base, tables, group, scratch), atol(p.atol), rtol(p.rtol), order(p.order) {}
+    __device__ Ctx(const Params& p, int g, double* lds)
+        : Base::Ctx(p.base, g, lds), atol(p.atol), rtol(p.rtol), order(p.order) {}
+    __device__ Ctx(const Params& p, const double* tables, double* group)
+        : Base::Ctx(p.base, tables, group), atol(p.atol), rtol(p.rtol), order(p.order) {}
   };
 
   template <int G, int R>

@@ -121,13 +121,12 @@ struct MechKinetics {
   //
   // per group: (C, gRT) pairs, hR, cpR [NS + 1 each]; kf, kr, q, qT [nr each]; the
   // Jacobian buffer [N*N] (d wdot / d C rows while the Jacobian is assembled,
-  // then the parked Jacobian); optionally a scratch [N*N] for integrators that
-  // transpose their factors through LDS.
-  __host__ __device__ static size_t group_doubles(int nr, bool scratch) {
-    return (size_t)4 * (NS + 1) + (size_t)4 * nr + (kLarge ? 0 : (size_t)(scratch ? 2 : 1) * N * N);
+  // then the parked Jacobian).
+  __host__ __device__ static size_t group_doubles(int nr) {
+    return (size_t)4 * (NS + 1) + (size_t)4 * nr + (kLarge ? 0 : (size_t)N * N);
   }
-  static size_t lds_bytes(const Params& p, int groups, bool scratch) {
-    return (size_t)p.lds_bytes + groups * group_doubles(p.nr, scratch) * sizeof(double);
+  static size_t lds_bytes(const Params& p, int groups) {
+    return (size_t)p.lds_bytes + groups * group_doubles(p.nr) * sizeof(double);
   }
 
   // Whole block: copy the network tables into LDS (before any divergence).
@@ -157,13 +156,12 @@ struct MechKinetics {
     double* q;
     double* qT;
     double* Jc;
-    double* scratch;
     double* jac;
     // tables copied by block_init at `lds`; group g's buffers after them
-    __device__ Ctx(const Params& pp, int g, double* lds, bool with_scratch)
-        : Ctx(pp, lds, lds + pp.lds_bytes / 8 + (size_t)g * group_doubles(pp.nr, with_scratch), with_scratch) {}
-    // tables at `tables`, the group's buffers at `group` (group_doubles(nr, with_scratch) doubles)
-    __device__ Ctx(const Params& pp, const double* tables, double* group, bool with_scratch)
+    __device__ Ctx(const Params& pp, int g, double* lds)
+        : Ctx(pp, lds, lds + pp.lds_bytes / 8 + (size_t)g * group_doubles(pp.nr)) {}
+    // tables at `tables`, the group's buffers at `group` (group_doubles(nr) doubles)
+    __device__ Ctx(const Params& pp, const double* tables, double* group)
         : nr(pp.nr), ell_batches(pp.ell_batches) {
       const char* t = reinterpret_cast<const char*>(tables);
       const char* gl = reinterpret_cast<const char*>(pp.blob);
@@ -186,12 +184,10 @@ struct MechKinetics {
       // d wdot / d C is fully consumed (column sums) before the caller parks
       // the Jacobian rows, so the two share one buffer
       if constexpr (kLarge) {
-        Jc = jac = scratch = nullptr;  // bind_global
+        Jc = jac = nullptr;  // bind_global
       } else {
         Jc = b;
         jac = b;
-        b += N * N;
-        scratch = with_scratch ? b : nullptr;
       }
     }
     // large networks: the parked Jacobian (kJacLd x N) and the d wdot / d C
@@ -380,8 +376,9 @@ struct MechKinetics {
   // c.jac[r*N + j] = d f_r / d y_j (row 0 = T).  The buffer doubles as the
   // d wdot / d C scratch, so each lane keeps its own d wdot / d C row in
   // registers until every lane has finished reading the scratch.  JB:
-  // incidence-list entries per batch (the caller's choice: a kernel whose
-  // FP64 factors already fill the register file runs it unbatched).
+  // incidence-list entries per batch (the caller's choice: only a 64-lane group
+  // with FP32 factors has the registers; FP64 factors fill the register file,
+  // and 16-lane groups run two waves per SIMD on half of it).
   static constexpr int kJacBatchFP32 = kKinJacBatch;
   static constexpr int kJacBatchFP64 = 1;
   template <int G, int R, int JB = kKinJacBatch>

@@ -42,13 +42,10 @@ struct MechUser {
   static constexpr bool kJacInLds = kUserG > 1;
   static constexpr bool kJacColMajor = true;
   struct Params {};
-  // per group: y, dy, the parameter, the Jacobian (N x N), and the column
-  // LU's transpose scratch when asked for
-  __host__ __device__ static size_t group_doubles(bool scratch) {
-    return kJacInLds ? (size_t)2 * N + 2 + (size_t)(scratch ? 2 : 1) * N * N : 0;
-  }
-  static size_t lds_bytes(const Params&, int groups, bool scratch) {
-    return (size_t)groups * group_doubles(scratch) * sizeof(double);
+  // per group: y, dy, the parameter and the Jacobian (N x N)
+  __host__ __device__ static size_t group_doubles() { return kJacInLds ? (size_t)2 * N + 2 + (size_t)N * N : 0; }
+  static size_t lds_bytes(const Params&, int groups) {
+    return (size_t)groups * group_doubles() * sizeof(double);
   }
   __device__ __forceinline__ static void block_init(const Params&, double*) {}
 
@@ -57,16 +54,13 @@ struct MechUser {
     double* dyb = nullptr;
     double* var = nullptr;
     double* jac = nullptr;
-    double* scratch = nullptr;
-    __device__ Ctx(const Params& p, int g, double* lds, bool with_scratch)
-        : Ctx(p, lds, lds + (size_t)g * group_doubles(with_scratch), with_scratch) {}
-    __device__ Ctx(const Params&, const double*, double* group, bool with_scratch) {
+    __device__ Ctx(const Params& p, int g, double* lds) : Ctx(p, lds, lds + (size_t)g * group_doubles()) {}
+    __device__ Ctx(const Params&, const double*, double* group) {
       if constexpr (kJacInLds) {
         yb = group;
         dyb = yb + N;
         var = dyb + N;
         jac = var + 2;
-        scratch = with_scratch ? jac + (size_t)N * N : nullptr;
       }
     }
   };

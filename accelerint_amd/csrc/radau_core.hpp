@@ -992,6 +992,10 @@ __device__ __forceinline__ int bcast_k_i(int v) {
   }
 }
 template <int G, int K>
+__device__ __forceinline__ float bcast_k(float v) {
+  return __int_as_float(bcast_k_i<G, K>(__float_as_int(v)));
+}
+template <int G, int K>
 __device__ __forceinline__ double bcast_k(double v) {
   if constexpr (G == 1) {
     return v;
@@ -1002,241 +1006,224 @@ __device__ __forceinline__ double bcast_k(double v) {
   }
 }
 
-// Packed original-row table for the explicit-interchange LU: byte i = the
-// original row now in position i.
-template <int N>
-struct RowMap {
-  uint32_t w[(N + 3) / 4];
-  __device__ __forceinline__ void init() {
-#pragma unroll
-    for (int i = 0; i < (N + 3) / 4; ++i) {
-      uint32_t v = 0;
-#pragma unroll
-      for (int b = 0; b < 4; ++b) v |= (uint32_t)((4 * i + b) & 0xff) << (8 * b);
-      w[i] = v;
-    }
-  }
-  __device__ __forceinline__ int get(int i) const {  // i may be a runtime value
-    uint32_t word = w[0];
-#pragma unroll
-    for (int q = 1; q < (N + 3) / 4; ++q) word = ((i >> 2) == q) ? w[q] : word;
-    return (int)((word >> (8 * (i & 3))) & 0xffu);
-  }
-  __device__ __forceinline__ void set(int i, int v) {  // runtime i
-    const int s = 8 * (i & 3);
-#pragma unroll
-    for (int q = 0; q < (N + 3) / 4; ++q)
-      if ((i >> 2) == q) w[q] = (w[q] & ~(0xffu << s)) | ((uint32_t)v << s);
-  }
-  __device__ __forceinline__ void swap(int i, int j) {
-    const int vi = get(i), vj = get(j);
-    set(i, vj);
-    set(j, vi);
-  }
-};
-
-// ---- column-layout LU (dgetf2 / zgetf2 with explicit interchanges) --------
-// Lane j of the group holds column j: a[i] = A(i, j).  For G >= N only.  The
-// pivot search of step k runs inside lane k (first maximum of |a| or
-// |Re|+|Im|, exactly LAPACK's idamax/izamax order since rows are physically
-// interchanged), the interchange is a register select in every lane, lane k
-// scales its column into multipliers and broadcasts them from a compile-time
-// lane.  On exit a[] holds LAPACK's combined L\U column, rmap the row
-// permutation, rdiag = 1/U(j, j) in lane j; info as LAPACK.
-template <int N, int G>
-__device__ __forceinline__ void clu_real(double (&a)[N], RowMap<N>& rmap, double& rdiag, int& info) {
-  static_assert(G >= N, "column LU needs a lane per column");
-  const int ln = Grp<G>::lane();
-  rmap.init();
-  info = 0;
-  rdiag = 0.0;
-  static_for<0, N>([&](auto kc) {
-    constexpr int k = decltype(kc)::value;
-    double vmax = fabs(a[k]);
-    int p = k;
-#pragma unroll
-    for (int i = k + 1; i < N; ++i) {
-      const double v = fabs(a[i]);
-      const bool gt = v > vmax;
-      vmax = gt ? v : vmax;
-      p = gt ? i : p;
-    }
-    const int code = bcast_k_i<G, k>(vmax != 0.0 ? p : (k | 0x100));
-    const bool nz = (code & 0x100) == 0;
-    p = code & 0xff;
-    if (!nz && info == 0) info = k + 1;
-    if (nz) rmap.swap(k, p);
-    // interchange rows k and p in every column
-    const double ak = a[k];
-    double ap = ak;
-#pragma unroll
-    for (int i = k + 1; i < N; ++i) ap = (i == p) ? a[i] : ap;
-#pragma unroll
-    for (int i = k + 1; i < N; ++i) a[i] = (i == p) ? ak : a[i];
-    a[k] = ap;
-    // lane k scales its column into multipliers (the other lanes scale by 1,
-    // which is exact).  LAPACK divides instead when |pivot| < DBL_MIN; that
-    // case only arises for subnormal pivots and is not reproduced.
-    const double rp = 1.0 / ap;
-    const bool mine = (ln == k) && nz;
-    if (ln == k) rdiag = nz ? rp : 0.0;
-    const double sf = mine ? rp : 1.0;
-#pragma unroll
-    for (int i = k + 1; i < N; ++i) a[i] *= sf;
-    // rank-1 update of the columns right of k
-    const double uk = (ln > k && ln < N) ? a[k] : 0.0;
-#pragma unroll
-    for (int i = k + 1; i < N; ++i) {
-      const double li = bcast_k<G, k>(a[i]);
-      a[i] = fma(-li, uk, a[i]);
-    }
-  });
+// ---- LU of 16-lane groups (N <= 16, a row per lane; four systems a wavefront) --
+// dgetf2 / zgetf2 semantics like the row LU above.  The pivot search exchanges
+// the leading 32 bits of the magnitudes inside the DPP row of the group (four
+// v_max_u32 with the exchange folded in) and reads the winner from the group's
+// 16 bits of one compare mask; rows that agree in those bits, which is rare, go
+// through the full (value, position) search.  The pivot row is in a lane that
+// differs from group to group, so its entries are gathered (ds_bpermute, all
+// columns of a step in flight behind the reciprocal).  At the end the rows move
+// to the lanes of their LAPACK positions, so that the solves broadcast from
+// compile-time lanes on the VALU.
+//
+// Bound by issue and the gathers' latency at two waves per SIMD.  It replaced a
+// lane-per-column LU (pivot search down a lane's registers, interchanges as
+// selects in every lane) of 58k cycles per FP64 pair at order 14, and in FP32
+// a row LU with gathered solves; measured on 262144 14-state conditions of two
+// steps: FP64 30.0 -> 17.3 ms, 30011 conditions of four steps with FP32 factors
+// 4.26 -> 3.40 ms (with the Jacobian's batches).
+__device__ __forceinline__ int bperm(int addr, int v) { return __builtin_amdgcn_ds_bpermute(addr, v); }
+__device__ __forceinline__ float bperm(int addr, float v) { return __int_as_float(bperm(addr, __float_as_int(v))); }
+__device__ __forceinline__ double bperm(int addr, double v) {
+  const int lo = bperm(addr, __double2loint(v)), hi = bperm(addr, __double2hiint(v));
+  return __hiloint2double(hi, lo);
 }
 
-template <int N, int G>
-__device__ __forceinline__ void clu_cplx(double (&ar)[N], double (&ai)[N], RowMap<N>& rmap,
-                                         double& rdr, double& rdi, int& info) {
-  static_assert(G >= N, "column LU needs a lane per column");
-  const int ln = Grp<G>::lane();
-  rmap.init();
-  info = 0;
-  rdr = 0.0;
-  rdi = 0.0;
-  static_for<0, N>([&](auto kc) {
-    constexpr int k = decltype(kc)::value;
-    double vmax = fabs(ar[k]) + fabs(ai[k]);
-    int p = k;
-#pragma unroll
-    for (int i = k + 1; i < N; ++i) {
-      const double v = fabs(ar[i]) + fabs(ai[i]);
-      const bool gt = v > vmax;
-      vmax = gt ? v : vmax;
-      p = gt ? i : p;
-    }
-    const int code = bcast_k_i<G, k>(vmax != 0.0 ? p : (k | 0x100));
-    const bool nz = (code & 0x100) == 0;
-    p = code & 0xff;
-    if (!nz && info == 0) info = k + 1;
-    if (nz) rmap.swap(k, p);
-    const double akr = ar[k], aki = ai[k];
-    double apr = akr, api = aki;
-#pragma unroll
-    for (int i = k + 1; i < N; ++i) {
-      apr = (i == p) ? ar[i] : apr;
-      api = (i == p) ? ai[i] : api;
-    }
-#pragma unroll
-    for (int i = k + 1; i < N; ++i) {
-      ar[i] = (i == p) ? akr : ar[i];
-      ai[i] = (i == p) ? aki : ai[i];
-    }
-    ar[k] = apr;
-    ai[k] = api;
-    double rr, ri;
-    crecip(apr, api, rr, ri);
-    const bool mine = (ln == k) && nz;
-    if (ln == k) {
-      rdr = nz ? rr : 0.0;
-      rdi = nz ? ri : 0.0;
-    }
-    // lane k scales by the reciprocal pivot, the others by 1 + 0i (exact)
-    const double sr = mine ? rr : 1.0, si = mine ? ri : 0.0;
-#pragma unroll
-    for (int i = k + 1; i < N; ++i) {
-      const double xr = ar[i], xi = ai[i];
-      ar[i] = xr * sr - xi * si;
-      ai[i] = xr * si + xi * sr;
-    }
-    const bool upd = ln > k && ln < N;
-    const double ukr = upd ? ar[k] : 0.0, uki = upd ? ai[k] : 0.0;
-#pragma unroll
-    for (int i = k + 1; i < N; ++i) {
-      const double lr = bcast_k<G, k>(ar[i]);
-      const double li = bcast_k<G, k>(ai[i]);
-      ar[i] = fma(-lr, ukr, ar[i]);
-      ar[i] = fma(li, uki, ar[i]);
-      ai[i] = fma(-lr, uki, ai[i]);
-      ai[i] = fma(-li, ukr, ai[i]);
-    }
-  });
+// Pivot row of a step: the lane of the group (first maximum of the magnitudes v
+// over the active rows in LAPACK's order pos), or 0xff if no active row holds a
+// comparable value.
+template <class T>
+__device__ __forceinline__ int row16_pivot(T v, int pos, bool act) {
+  const unsigned key = act && v == v ? mag_hi(v) + 1u : 0u;  // 0: no candidate
+  unsigned m = dpp_max_u<kDppXor1>(key);
+  m = dpp_max_u<kDppXor2>(m);
+  m = dpp_max_u<kDppHalfMirror>(m);
+  m = dpp_max_u<kDppMirror>(m);
+  const unsigned long long all = __builtin_amdgcn_ballot_w64(key == m);
+  const int lane = (int)__lane_id();
+  const unsigned half = (lane & 32) ? (unsigned)(all >> 32) : (unsigned)all;
+  const unsigned cand = (half >> (lane & 16)) & 0xffffu;
+  int prow = __builtin_ctz(cand | 0x10000u);
+  if (__builtin_expect((cand & (cand - 1)) != 0, 0)) {
+    T bv = act && v == v ? v : T(-1);
+    int bkey = act && v == v ? ((pos << 8) | (lane & 15)) : 0x7fffffff;
+    group_argmax<16>(bv, bkey);
+    prow = bkey & 0xff;
+  }
+  return prow;
 }
 
-// Column layout (lane j holds column j) -> row layout (lane i holds row i) of
-// an N x N block through the group's LDS scratch (N*N doubles).
-template <int N, int G>
-__device__ __forceinline__ void transpose_cols_to_rows(const double (&col)[N], double (&row)[N],
-                                                       double* scratch) {
-  const int ln = Grp<G>::lane();
-  if (ln < N) {
+// Rows to the lanes of their positions: src = the row (lane) whose position is
+// this lane's index.
+__device__ __forceinline__ int row16_source(int pos) {
+  const int lane = (int)__lane_id(), base = lane & 48;
+  const int to = pos >= 0 ? (pos & 15) : (lane & 15);
+  return __builtin_amdgcn_ds_permute((base | to) << 2, lane & 15) & 15;
+}
+
+template <int N, class T>
+__device__ __forceinline__ void row16_lu_real(T (&a)[N], int& src, T& rd, int& info) {
+  static_assert(N <= 16, "a 16-lane group holds at most 16 rows");
+  const int ln = Grp<16>::lane(), base = (int)__lane_id() & 48;
+  int pos = ln < N ? ln : -1;
+  rd = T(0);
+  info = 0;
 #pragma unroll
-    for (int i = 0; i < N; ++i) scratch[i * N + ln] = col[i];
+  for (int k = 0; k < N; ++k) {
+    const int prow = row16_pivot(fabs(a[k]), pos, pos >= k);
+    const int from = (base | (prow & 15)) << 2;
+    const int ppos = prow == 0xff ? 0x7fffff : bperm(from, pos);
+    const T piv = bperm(from, a[k]);
+    T u[N];
+#pragma unroll
+    for (int j = k + 1; j < N; ++j) u[j] = bperm(from, a[j]);
+    const bool is_piv = ln == prow;
+    pos = is_piv ? k : (pos == k ? ppos : pos);
+    pin(pos);
+    const bool nz = piv != T(0);
+    info = !nz && info == 0 ? k + 1 : info;
+    pin(info);
+    const T rp = recip(piv);
+    T lq = a[k] * rp;
+    if constexpr (std::is_same<T, double>::value)
+      if (__builtin_expect(fabs(piv) < min_normal<T>(), 0)) lq = a[k] / piv;
+    rd = is_piv ? (nz ? rp : T(0)) : rd;
+    pin(rd);
+    const bool act = nz && pos > k;
+    a[k] = act ? lq : a[k];
+    T l = act ? -lq : T(-0.0);
+    pin(a[k]);
+    pin(l);
+#pragma unroll
+    for (int j = k + 1; j < N; ++j) {
+      a[j] = fma(l, u[j], a[j]);
+      pin(a[j]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
   }
-  __asm__ volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt(0xC07F);
-  __builtin_amdgcn_wave_barrier();
-  __asm__ volatile("" ::: "memory");
+  src = row16_source(pos);
+  const int from = (base | src) << 2;
 #pragma unroll
-  for (int j = 0; j < N; ++j) row[j] = (ln < N) ? scratch[ln * N + j] : 0.0;
-  __asm__ volatile("" ::: "memory");
-  __builtin_amdgcn_s_waitcnt(0xC07F);
-  __builtin_amdgcn_wave_barrier();
-  __asm__ volatile("" ::: "memory");
+  for (int j = 0; j < N; ++j) a[j] = bperm(from, a[j]);
+  rd = bperm(from, rd);
+}
+
+template <int N, class T>
+__device__ __forceinline__ void row16_lu_cplx(T (&ar)[N], T (&ai)[N], int& src, T& rdr, T& rdi, int& info) {
+  static_assert(N <= 16, "a 16-lane group holds at most 16 rows");
+  const int ln = Grp<16>::lane(), base = (int)__lane_id() & 48;
+  int pos = ln < N ? ln : -1;
+  rdr = rdi = T(0);
+  info = 0;
+#pragma unroll
+  for (int k = 0; k < N; ++k) {
+    const int prow = row16_pivot(fabs(ar[k]) + fabs(ai[k]), pos, pos >= k);
+    const int from = (base | (prow & 15)) << 2;
+    const int ppos = prow == 0xff ? 0x7fffff : bperm(from, pos);
+    const T pr_ = bperm(from, ar[k]), pi_ = bperm(from, ai[k]);
+    T ur[N], ui[N];
+#pragma unroll
+    for (int j = k + 1; j < N; ++j) {
+      ur[j] = bperm(from, ar[j]);
+      ui[j] = bperm(from, ai[j]);
+    }
+    const bool is_piv = ln == prow;
+    pos = is_piv ? k : (pos == k ? ppos : pos);
+    pin(pos);
+    const bool nz = pr_ != T(0) || pi_ != T(0);
+    info = !nz && info == 0 ? k + 1 : info;
+    pin(info);
+    T rr, ri;
+    crecip(pr_, pi_, rr, ri);
+    rdr = is_piv ? (nz ? rr : T(0)) : rdr;
+    rdi = is_piv ? (nz ? ri : T(0)) : rdi;
+    pin(rdr);
+    pin(rdi);
+    const bool act = nz && pos > k;
+    const T xr = ar[k], xi = ai[k];
+    const T vr = xr * rr - xi * ri;
+    const T vi = xr * ri + xi * rr;
+    ar[k] = act ? vr : xr;
+    ai[k] = act ? vi : xi;
+    T lr = act ? vr : T(0), li = act ? vi : T(0);
+    pin(ar[k]);
+    pin(ai[k]);
+    pin(lr);
+    pin(li);
+#pragma unroll
+    for (int j = k + 1; j < N; ++j) {
+      ar[j] = fma(li, ui[j], fma(-lr, ur[j], ar[j]));
+      ai[j] = fma(-li, ur[j], fma(-lr, ui[j], ai[j]));
+      pin(ar[j]);
+      pin(ai[j]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  src = row16_source(pos);
+  const int from = (base | src) << 2;
+#pragma unroll
+  for (int j = 0; j < N; ++j) {
+    ar[j] = bperm(from, ar[j]);
+    ai[j] = bperm(from, ai[j]);
+  }
+  rdr = bperm(from, rdr);
+  rdi = bperm(from, rdi);
 }
 
 // ---- row-layout solves for the explicit-interchange factors ----------------
-// Lane i holds row i of L\U (LAPACK order) and src = the original row whose
-// equation sits in position i; b[] is the right-hand side of the lane's own
+// 16-lane groups: lane i holds row i of L\U (LAPACK order) and src = the original
+// row whose equation sits in position i; b[] is the right-hand side of the lane's own
 // (original) equation.  Pivot rows are at compile-time lanes, so every
 // broadcast comes from a fixed lane.  On return b holds solution component i
 // in lane i.
-template <int N, int G>
-__device__ __forceinline__ void rsolve_real(const double (&a)[N], int src, double rdiag,
-                                            double& b) {
-  const int ln = Grp<G>::lane();
-  double x = Grp<G>::gather(b, src);  // (P b)_i
+// (The triangles are masked by compile-time steps against the lane, so the
+// coefficients are taken as they are and the rows outside a step keep x by a
+// select: see SolveView.)
+template <int N, int G, class T>
+__device__ __forceinline__ void rsolve_real(const T (&a)[N], int src, T rdiag, T& b) {
+  int ln = Grp<G>::lane();
+  pin(ln);
+  T x = __shfl(b, src, G);  // (P b)_i
   static_for<0, N>([&](auto kc) {
     constexpr int k = decltype(kc)::value;
-    const double yk = bcast_k<G, k>(x);
-    x = fma(-(ln > k && ln < N ? a[k] : 0.0), yk, x);
+    const T v = fma(-a[k], bcast_k<G, k>(x), x);
+    x = ln > k && ln < N ? v : x;
   });
   static_for<0, N>([&](auto kc) {
     constexpr int k = N - 1 - decltype(kc)::value;
-    const double xk = bcast_k<G, k>(x * rdiag);
-    if (ln == k) x = xk;
-    x = fma(-(ln < k ? a[k] : 0.0), xk, x);
+    const T xk = bcast_k<G, k>(x * rdiag);
+    const T v = fma(-a[k], xk, x);
+    x = ln < k ? v : (ln == k ? xk : x);
   });
-  b = (ln < N) ? x : 0.0;
+  b = (ln < N) ? x : T(0);
 }
 
-template <int N, int G>
-__device__ __forceinline__ void rsolve_cplx(const double (&ar)[N], const double (&ai)[N], int src,
-                                            double rdr, double rdi, double& br, double& bi) {
-  const int ln = Grp<G>::lane();
-  double xr = Grp<G>::gather(br, src), xi = Grp<G>::gather(bi, src);
+template <int N, int G, class T>
+__device__ __forceinline__ void rsolve_cplx(const T (&ar)[N], const T (&ai)[N], int src, T rdr, T rdi, T& br, T& bi) {
+  int ln = Grp<G>::lane();
+  pin(ln);
+  T xr = __shfl(br, src, G), xi = __shfl(bi, src, G);
   static_for<0, N>([&](auto kc) {
     constexpr int k = decltype(kc)::value;
-    const double yr = bcast_k<G, k>(xr), yi = bcast_k<G, k>(xi);
+    const T yr = bcast_k<G, k>(xr), yi = bcast_k<G, k>(xi);
     const bool act = ln > k && ln < N;
-    const double lr = act ? ar[k] : 0.0, li = act ? ai[k] : 0.0;
-    xr = fma(-lr, yr, xr);
-    xr = fma(li, yi, xr);
-    xi = fma(-lr, yi, xi);
-    xi = fma(-li, yr, xi);
+    const T vr = fma(ai[k], yi, fma(-ar[k], yr, xr));
+    const T vi = fma(-ai[k], yr, fma(-ar[k], yi, xi));
+    xr = act ? vr : xr;
+    xi = act ? vi : xi;
   });
   static_for<0, N>([&](auto kc) {
     constexpr int k = N - 1 - decltype(kc)::value;
-    const double kr = bcast_k<G, k>(xr * rdr - xi * rdi);
-    const double ki = bcast_k<G, k>(xr * rdi + xi * rdr);
-    if (ln == k) { xr = kr; xi = ki; }
-    const bool act = ln < k;
-    const double ur = act ? ar[k] : 0.0, ui = act ? ai[k] : 0.0;
-    xr = fma(-ur, kr, xr);
-    xr = fma(ui, ki, xr);
-    xi = fma(-ur, ki, xi);
-    xi = fma(-ui, kr, xi);
+    const T kr = bcast_k<G, k>(xr * rdr - xi * rdi);
+    const T ki = bcast_k<G, k>(xr * rdi + xi * rdr);
+    const T vr = fma(ai[k], ki, fma(-ar[k], kr, xr));
+    const T vi = fma(-ai[k], kr, fma(-ar[k], ki, xi));
+    xr = ln < k ? vr : (ln == k ? kr : xr);
+    xi = ln < k ? vi : (ln == k ? ki : xi);
   });
-  br = (ln < N) ? xr : 0.0;
-  bi = (ln < N) ? xi : 0.0;
+  br = (ln < N) ? xr : T(0);
+  bi = (ln < N) ? xi : T(0);
 }
 
 // ---- the integrator ----------------------------------------------------------
@@ -1280,14 +1267,9 @@ struct Radau {
   // error estimate, step control and state in FP64).
   static constexpr bool kMixed = std::is_same<MT, float>::value;
   static_assert(kMixed || std::is_same<MT, double>::value, "matrix type must be float or double");
-  // Column-layout LU with compile-time broadcast lanes when one lane per
-  // column fits in a DPP row (G = 16) and the Jacobian is parked in LDS (it is
-  // read back column-wise); implicit-pivot row LU otherwise.  At G = 64 the
-  // row LU broadcasts pivot rows through SGPRs (readlane), which is cheaper
-  // than the column form's interchange selects.
-  static constexpr bool kColLU = G == 16 && G >= N && R == 1 && Mech::kJacInLds && !kMixed;
-  // The column LU transposes its factors through a per-group LDS scratch.
-  static constexpr bool kNeedsScratch = kColLU;
+  // 16-lane groups: the row LU that ends with every row in the lane of its
+  // position (row16_lu_*), and solves with compile-time broadcast lanes.
+  static constexpr bool kRow16 = G == 16 && R == 1;
   // Systems above 64 states: a wavefront per condition (R rows per lane), the
   // factorizations in a per-wave global workspace (MemLU: blocked LU with
   // MFMA trailing updates) instead of registers.
@@ -1337,7 +1319,7 @@ struct Radau {
   __device__ __forceinline__ int row_exp2(int q) const { return kMemLU ? ex2[q] : ex1[q] >> 16; }
   MT rd1[R], rd2r[R], rd2i[R];
   Perm<N> perm1, perm2;
-  int src1, src2;  // column-LU path: original equation of this lane's row
+  int src1, src2;  // 16-lane groups: original equation of this lane's row
   double A[R][N];  // Jacobian (only live across attempts when !Mech::kJacInLds)
   // predicted Newton start of the current global step's first step; dropped
   // (zero start, the reference's rule) after any rejection of that step
@@ -1375,8 +1357,10 @@ struct Radau {
       MLU::solve_real(wE1(), wipiv1(), bb);
 #pragma unroll
       for (int q = 0; q < R; ++q) b[q] = kMixed ? ldexp((double)bb[q], -cx1[q]) : (double)bb[q];
-    } else if constexpr (kColLU) {
-      rsolve_real<N, G>(E1[0], src1, rd1[0], b[0]);
+    } else if constexpr (kRow16) {
+      MT x = kMixed ? (MT)ldexp(b[0], -row_exp1(0)) : (MT)b[0];
+      rsolve_real<N, G, MT>(E1[0], src1, rd1[0], x);
+      b[0] = kMixed ? ldexp((double)x, -cx1[0]) : (double)x;
     } else if constexpr (!kMixed) {
       solve_real<N, G, R, double>(E1, pos1, perm1, rd1, b);
     } else {
@@ -1402,8 +1386,12 @@ struct Radau {
         br[q] = kMixed ? ldexp((double)xr[q], -cx2[q]) : (double)xr[q];
         bi[q] = kMixed ? ldexp((double)xi[q], -cx2[q]) : (double)xi[q];
       }
-    } else if constexpr (kColLU) {
-      rsolve_cplx<N, G>(E2r[0], E2i[0], src2, rd2r[0], rd2i[0], br[0], bi[0]);
+    } else if constexpr (kRow16) {
+      MT xr = kMixed ? (MT)ldexp(br[0], -row_exp2(0)) : (MT)br[0];
+      MT xi = kMixed ? (MT)ldexp(bi[0], -row_exp2(0)) : (MT)bi[0];
+      rsolve_cplx<N, G, MT>(E2r[0], E2i[0], src2, rd2r[0], rd2i[0], xr, xi);
+      br[0] = kMixed ? ldexp((double)xr, -cx1[0]) : (double)xr;
+      bi[0] = kMixed ? ldexp((double)xi, -cx1[0]) : (double)xi;
     } else if constexpr (!kMixed) {
       solve_cplx<N, G, R, double>(E2r, E2i, pos2, perm2, rd2r, rd2i, br, bi);
     } else {
@@ -1624,91 +1612,73 @@ struct Radau {
     const int ln = Grp<G>::lane();
     const double g1 = rkGamma / H, g2r = rkAlpha / H, g2i = rkBeta / H;
     int info = 0, info2 = 0;
-    if constexpr (kColLU) {
-      group_lds_sync();  // the parked Jacobian rows of all lanes
-      double c1[N], c2r[N], c2i[N];
+    if constexpr (Mech::kJacInLds) group_lds_sync();
+    auto jac_at = [&](int q, int r, int j) -> double {
+      if constexpr (Mech::kJacInLds) return jac_entry(ctx, ln, q, j);
+      else return A[q][j];
+    };
+    if constexpr (kMixed && kMemLU) {
+      equilibrate(jac_at, g1, 0.0, ex1, cx1);
+      equilibrate(jac_at, g2r, g2i, ex2, cx2);
+    } else if constexpr (kMixed) {
+      int e1[R], e2[R];
+      row_exponents(jac_at, g1, 0.0, e1);
+      row_exponents(jac_at, g2r, g2i, e2);
 #pragma unroll
-      for (int i = 0; i < N; ++i) {
-        const double jij = (ln < N) ? ctx.jac[jidx<Mech>(i, ln)] : 0.0;
-        const bool d = (i == ln);
-        c1[i] = -jij + (d ? g1 : 0.0);
-        c2r[i] = -jij + (d ? g2r : 0.0);
-        c2i[i] = d ? g2i : 0.0;
-      }
-      RowMap<N> m1, m2;
-      clu_real<N, G>(c1, m1, rd1[0], info);
-      transpose_cols_to_rows<N, G>(c1, E1[0], ctx.scratch);
-      src1 = m1.get(ln);
-      clu_cplx<N, G>(c2r, c2i, m2, rd2r[0], rd2i[0], info2);
-      transpose_cols_to_rows<N, G>(c2r, E2r[0], ctx.scratch);
-      transpose_cols_to_rows<N, G>(c2i, E2i[0], ctx.scratch);
-      src2 = m2.get(ln);
-    } else {
-      if constexpr (Mech::kJacInLds) group_lds_sync();
-      auto jac_at = [&](int q, int r, int j) -> double {
-        if constexpr (Mech::kJacInLds) return jac_entry(ctx, ln, q, j);
-        else return A[q][j];
-      };
-      if constexpr (kMixed && kMemLU) {
-        equilibrate(jac_at, g1, 0.0, ex1, cx1);
-        equilibrate(jac_at, g2r, g2i, ex2, cx2);
-      } else if constexpr (kMixed) {
-        int e1[R], e2[R];
-        row_exponents(jac_at, g1, 0.0, e1);
-        row_exponents(jac_at, g2r, g2i, e2);
+      for (int q = 0; q < R; ++q) ex1[q] = (int)(((unsigned)e1[q] & 0xffffu) | ((unsigned)e2[q] << 16));
+    }
+    // entry (r, j) of a matrix scaled by 2^-(e + c_j): c_j is held by the
+    // lane that holds row j
+    auto scaled = [&](double v, int e, int cj) -> MT { return kMixed ? (MT)ldexp(v, -(e + cj)) : (MT)v; };
 #pragma unroll
-        for (int q = 0; q < R; ++q) ex1[q] = (int)(((unsigned)e1[q] & 0xffffu) | ((unsigned)e2[q] << 16));
-      }
-      // entry (r, j) of a matrix scaled by 2^-(e + c_j): c_j is held by the
-      // lane that holds row j
-      auto scaled = [&](double v, int e, int cj) -> MT { return kMixed ? (MT)ldexp(v, -(e + cj)) : (MT)v; };
-#pragma unroll
-      for (int q = 0; q < R; ++q) {
-        const int r = RW::row(ln, q);
-        const int e1 = kMixed ? row_exp1(q) : 0, e2 = kMixed ? row_exp2(q) : 0;
-        if constexpr (kMemLU) {
-          MT* w1 = wE1() + r;
-          MT* w2r = wE2r() + r;
-          MT* w2i = wE2i() + r;
+    for (int q = 0; q < R; ++q) {
+      const int r = RW::row(ln, q);
+      const int e1 = kMixed ? row_exp1(q) : 0, e2 = kMixed ? row_exp2(q) : 0;
+      if constexpr (kMemLU) {
+        MT* w1 = wE1() + r;
+        MT* w2r = wE2r() + r;
+        MT* w2i = wE2i() + r;
 #pragma unroll 4
-          for (int j = 0; j < N; ++j) {
-            // the column exponents are read across lanes (readlane), so with
-            // every lane active: inside a branch on the row's validity the
-            // lanes holding rows beyond N would not have computed them
-            const int c1 = kMixed ? col_exp(cx1, j) : 0, c2 = kMixed ? col_exp(cx2, j) : 0;
-            const bool d = (j == r);
-            const double aj = jac_at(q, r, j);
-            if (RW::valid(ln, q)) {
-              w1[(size_t)j * MLU::LD] = scaled(-aj + (d ? g1 : 0.0), e1, c1);
-              w2r[(size_t)j * MLU::LD] = scaled(-aj + (d ? g2r : 0.0), e2, c2);
-              w2i[(size_t)j * MLU::LD] = scaled(d ? g2i : 0.0, e2, c2);
-            }
-          }
-        } else {
-          // (mixed: J' is column-scaled already; the diagonal takes its own
-          // column's scale)
-          const double d1 = kMixed ? ldexp(g1, -cx1[q]) : g1;
-          const double d2r = kMixed ? ldexp(g2r, -cx1[q]) : g2r, d2i = kMixed ? ldexp(g2i, -cx1[q]) : g2i;
-#pragma unroll
-          for (int j = 0; j < N; ++j) {
-            const bool d = (j == r);
-            const double aj = jac_at(q, r, j);
-            E1[q][j] = scaled(-aj + (d ? d1 : 0.0), e1, 0);
-            E2r[q][j] = scaled(-aj + (d ? d2r : 0.0), e2, 0);
-            E2i[q][j] = scaled(d ? d2i : 0.0, e2, 0);
+        for (int j = 0; j < N; ++j) {
+          // the column exponents are read across lanes (readlane), so with
+          // every lane active: inside a branch on the row's validity the
+          // lanes holding rows beyond N would not have computed them
+          const int c1 = kMixed ? col_exp(cx1, j) : 0, c2 = kMixed ? col_exp(cx2, j) : 0;
+          const bool d = (j == r);
+          const double aj = jac_at(q, r, j);
+          if (RW::valid(ln, q)) {
+            w1[(size_t)j * MLU::LD] = scaled(-aj + (d ? g1 : 0.0), e1, c1);
+            w2r[(size_t)j * MLU::LD] = scaled(-aj + (d ? g2r : 0.0), e2, c2);
+            w2i[(size_t)j * MLU::LD] = scaled(d ? g2i : 0.0, e2, c2);
           }
         }
-      }
-      if constexpr (kMemLU) {
-        wave_vmem_sync();  // every lane's rows before the panels read them
-        MLU::factor_real(wE1(), wipiv1(), info);
-        MLU::factor_cplx(wE2r(), wE2i(), wipiv2(), info2);
       } else {
-        // (interleaving the two factorizations' steps was measured slower at
-        // N = 54: the larger live set spills)
-        lu_real<N, G, R, MT>(E1, pos1, perm1, rd1, info);
-        lu_cplx<N, G, R, MT>(E2r, E2i, pos2, perm2, rd2r, rd2i, info2);
+        // (mixed: J' is column-scaled already; the diagonal takes its own
+        // column's scale)
+        const double d1 = kMixed ? ldexp(g1, -cx1[q]) : g1;
+        const double d2r = kMixed ? ldexp(g2r, -cx1[q]) : g2r, d2i = kMixed ? ldexp(g2i, -cx1[q]) : g2i;
+#pragma unroll
+        for (int j = 0; j < N; ++j) {
+          const bool d = (j == r);
+          const double aj = jac_at(q, r, j);
+          E1[q][j] = scaled(-aj + (d ? d1 : 0.0), e1, 0);
+          E2r[q][j] = scaled(-aj + (d ? d2r : 0.0), e2, 0);
+          E2i[q][j] = scaled(d ? d2i : 0.0, e2, 0);
+        }
       }
+    }
+    if constexpr (kMemLU) {
+      wave_vmem_sync();  // every lane's rows before the panels read them
+      MLU::factor_real(wE1(), wipiv1(), info);
+      MLU::factor_cplx(wE2r(), wE2i(), wipiv2(), info2);
+    } else if constexpr (kRow16) {
+      row16_lu_real<N, MT>(E1[0], src1, rd1[0], info);
+      row16_lu_cplx<N, MT>(E2r[0], E2i[0], src2, rd2r[0], rd2i[0], info2);
+    } else {
+      // (interleaving the two factorizations' steps was measured slower at
+      // N = 54: the larger live set spills)
+      lu_real<N, G, R, MT>(E1, pos1, perm1, rd1, info);
+      lu_cplx<N, G, R, MT>(E2r, E2i, pos2, perm2, rd2r, rd2i, info2);
     }
     return info != 0 ? info : info2;
   }
@@ -1791,7 +1761,7 @@ struct Radau {
       if (!SkipJac) {
         if constexpr (Mech::kJacInLds) {
           if constexpr (JacBatched<Mech>::value)
-            Mech::template jacob<G, R, kMixed ? Mech::kJacBatchFP32 : Mech::kJacBatchFP64>(ctx, t, pr, y);
+            Mech::template jacob<G, R, kMixed && G == 64 ? Mech::kJacBatchFP32 : Mech::kJacBatchFP64>(ctx, t, pr, y);
           else
             Mech::template jacob<G, R>(ctx, t, pr, y);
         } else {

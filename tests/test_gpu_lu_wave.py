@@ -1,5 +1,6 @@
-"""Pivot search of the one-wavefront LU (order 54) on candidates that agree in
-their leading 32 bits: the search compares those first and the rest only among
+"""Pivot search of the one-wavefront LU (order 54) and of the 16-lane groups' LU
+(order 14, four matrices a wavefront) on candidates that agree in their leading
+32 bits: the search compares those first and the rest only among
 the rows that attain the maximum.  Interchanges must be the oracle's dgetrf /
 zgetrf ones: the largest magnitude wins whichever bits decide it, and equal
 magnitudes go to the first row in LAPACK's current order.
@@ -11,7 +12,7 @@ import accelerint_amd as acc
 
 pytestmark = pytest.mark.gpu
 
-N = 54
+STEPS = [(54, 0), (54, 1), (54, 17), (54, 52), (14, 0), (14, 1), (14, 5), (14, 12)]
 
 
 @pytest.fixture
@@ -21,7 +22,7 @@ def session():
     acc.cleanup()
 
 
-def embedded(rng, k, column):
+def embedded(rng, N, k, column):
     """Order-N matrix whose step-k candidates are `column` (N - k values): a
     well-separated leading block first, rows of it shuffled so that the steps
     before k have interchanged rows."""
@@ -36,13 +37,13 @@ def embedded(rng, k, column):
 
 
 @pytest.mark.parametrize("cplx", [False, True])
-@pytest.mark.parametrize("k", [0, 1, 17, 52])
-def test_low_bits_decide(session, oracle_lib, k, cplx):
+@pytest.mark.parametrize("N,k", STEPS)
+def test_low_bits_decide(session, oracle_lib, N, k, cplx):
     rng = np.random.default_rng(90 + k)
     mats = []
-    for spread in (1, 3, 40):  # how many candidates share each value
+    for spread in (1, 3, 40, 1, 2):  # how many candidates share each value
         c = 1.0 + (rng.permutation(N - k) // spread) * 2.0 ** -50
-        mats.append(embedded(rng, k, c * rng.choice([-1.0, 1.0], N - k)))
+        mats.append(embedded(rng, N, k, c * rng.choice([-1.0, 1.0], N - k)))
     a = np.array(mats)
     if cplx:  # pure real and pure imaginary candidates of one magnitude rule
         a = a * np.where(rng.random((len(mats), N, 1)) < 0.5, 1.0, 1.0j)
@@ -53,10 +54,10 @@ def test_low_bits_decide(session, oracle_lib, k, cplx):
         assert np.array_equal(ipiv[m], f(a[m])[1])
 
 
-@pytest.mark.parametrize("k", [0, 1, 17, 52])
-def test_equal_candidates_fp32(session, oracle_lib, k):
+@pytest.mark.parametrize("N,k", STEPS)
+def test_equal_candidates_fp32(session, oracle_lib, N, k):
     rng = np.random.default_rng(190 + k)
-    a = embedded(rng, k, rng.choice([-1.0, 1.0], N - k))
+    a = embedded(rng, N, k, rng.choice([-1.0, 1.0], N - k))
     a = a.astype(np.float32).astype(np.float64)[None]
     _, ipiv, info = acc.factor_test(a, acc.PRECISION_MIXED)
     assert info[0] == 0
