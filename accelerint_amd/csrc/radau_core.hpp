@@ -91,6 +91,7 @@ constexpr double rkTiAi21 = 5.895975725255405108079130152868952;
 constexpr double rkTiAi22 = -1.441236197545344702389881889085515e-1;
 constexpr double rkELO = 4.0;
 
+
 // Return codes: radau2a/radau2a_props.h:30-39.
 enum : int {
   EC_success = 0,
@@ -178,6 +179,7 @@ struct Grp {
   // two sums side by side: the same operations as two calls of sum, their
   // dependent chains overlapped
   __device__ __forceinline__ static void sum2(double& a, double& b);
+  __device__ __forceinline__ static void sum3(double& a, double& b, double& c);
 };
 
 // Row ownership helpers.
@@ -262,15 +264,14 @@ __device__ __forceinline__ void crecip(T c, T d, T& re, T& im) {
     re = cd ? iden : r * iden;
     im = cd ? -r * iden : -iden;
   } else {
-    if (fabs(c) >= fabs(d)) {
-      T r = d / c, den = c + d * r;
-      re = T(1) / den;
-      im = -r / den;
-    } else {
-      T r = c / d, den = c * r + d;
-      re = r / den;
-      im = T(-1) / den;
-    }
+    // selected operands, not branches: in lane groups narrower than a wavefront
+    // both sides would run, and the two quotients overlap
+    const bool cd = fabs(c) >= fabs(d);
+    const T a = cd ? c : d, b = cd ? d : c;
+    const T r = b / a, den = a + b * r;
+    const T iden = T(1) / den, rden = r / den;
+    re = cd ? iden : rden;
+    im = cd ? -rden : -iden;
   }
 }
 
@@ -511,6 +512,37 @@ __device__ __forceinline__ void Grp<G>::sum2(double& a, double& b) {
   } else {
     a = sum(a);
     b = sum(b);
+  }
+}
+
+template <int G>
+__device__ __forceinline__ void Grp<G>::sum3(double& a, double& b, double& c) {
+  if constexpr (G == 16 || G == 64) {
+    double x = dpp_t<kDppXor1>(a), z = dpp_t<kDppXor1>(b), w = dpp_t<kDppXor1>(c);
+    a += x;
+    b += z;
+    c += w;
+    x = dpp_t<kDppXor2>(a), z = dpp_t<kDppXor2>(b), w = dpp_t<kDppXor2>(c);
+    a += x;
+    b += z;
+    c += w;
+    x = dpp_t<kDppHalfMirror>(a), z = dpp_t<kDppHalfMirror>(b), w = dpp_t<kDppHalfMirror>(c);
+    a += x;
+    b += z;
+    c += w;
+    x = dpp_t<kDppMirror>(a), z = dpp_t<kDppMirror>(b), w = dpp_t<kDppMirror>(c);
+    a += x;
+    b += z;
+    c += w;
+    if constexpr (G == 64) {
+      a = (bcast(a, 0) + bcast(a, 16)) + (bcast(a, 32) + bcast(a, 48));
+      b = (bcast(b, 0) + bcast(b, 16)) + (bcast(b, 32) + bcast(b, 48));
+      c = (bcast(c, 0) + bcast(c, 16)) + (bcast(c, 32) + bcast(c, 48));
+    }
+  } else {
+    a = sum(a);
+    b = sum(b);
+    c = sum(c);
   }
 }
 
@@ -1251,10 +1283,61 @@ enum : int { RADAU_CONTINUE = -1 };
 #include "lu_mem.hpp"
 namespace acc {
 
-// pow as a real call.  The step controller calls it at five places where all
-// of the integrator's state is live; inlined, the library routine's many
-// temporaries push the register allocation into spills around every site.
-// Out of line it returns the same values at the cost of a call.
+// The step controller's powers.  pow() itself is ~250 instructions, called two to
+// four times per attempt with all of the integrator's state live (a third of a
+// van der Pol attempt); the exponents that occur every time are fixed, so they
+// take Newton's iteration on the root from a hardware FP32 start (relative error
+// 1e-6, squared twice): 15 instructions, inline.  Largest error over the ranges
+// below, 1e7 arguments each against 80-bit arithmetic, in units of 2^-53:
+// inv_root4 1.60 (pow 1.98), pow_0p8 2.24, pow_int 1.99.  With the norms' shared
+// root and the quotients by H and by constants from one reciprocal (quot):
+// 262144 oscillators of five steps 0.82 -> 0.58 ms, 262144 14-state conditions of
+// two steps 17.3 -> 15.7 ms (FP64), 65536 54-state ones with FP32 factors
+// 162.1 -> 157.6 ms.
+//
+// x^(-1/4), x > 0; arguments above 1e38 count as 1e38 (the controller's factors
+// are clamped long before).
+__device__ __forceinline__ double inv_root4(double x) {
+  x = fmin(x, 1e38);
+  double y = (double)__builtin_amdgcn_rsqf(__builtin_amdgcn_sqrtf((float)x));
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {  // y += y (1 - x y^4) / 4
+    const double y2 = y * y;
+    y = fma(y, 0.25 * fma(-(x * y2), y2, 1.0), y);
+  }
+  return y;
+}
+// x^0.8 = x x^(-1/5), 1e-16 <= x <= 1e3 (the Newton rate).
+__device__ __forceinline__ double pow_0p8(double x) {
+  double y = (double)__builtin_amdgcn_exp2f(-0.2f * __builtin_amdgcn_logf((float)x));
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {  // y += y (1 - x y^5) / 5
+    const double y2 = y * y;
+    y = fma(y, 0.2 * fma(-(x * y), y2 * y2, 1.0), y);
+  }
+  return x * y;
+}
+// x^n, 0 <= n <= 7, the products' rounding errors carried along.
+__device__ __forceinline__ double pow_int(double x, int n) {
+  const double x2 = x * x, e2 = fma(x, x, -x2);
+  const double x4 = x2 * x2, e4 = fma(x2, x2, -x4) + 2.0 * x2 * e2;
+  double p = (n & 1) ? x : 1.0, e = 0.0;
+  const double p2 = p * x2, f2 = fma(p, x2, -p2) + p * e2;
+  p = (n & 2) ? p2 : p;
+  e = (n & 2) ? f2 : e;
+  const double p4 = p * x4, f4 = fma(p, x4, -p4) + (p * e4 + e * x4);
+  return (n & 4) ? p4 + f4 : p + e;
+}
+// x / d from the reciprocal id = 1 / d: the product corrected by its residual,
+// which gives the quotient's rounding (all but exceptional last bits) in three
+// instructions instead of a division's eleven.
+__device__ __forceinline__ double quot(double x, double d, double id) {
+  const double q = x * id;
+  return fma(fma(-q, d, x), id, q);
+}
+// The step factor of a failing Newton iteration has an exponent that depends on
+// the iteration: pow as a real call, so that its temporaries stay out of the
+// integrator's register allocation (inlined, they spilled around the site).
 __device__ __attribute__((noinline)) inline double step_pow(double x, double y) { return pow(x, y); }
 
 template <class Mech, int G, int R, class MT = double>
@@ -1610,7 +1693,8 @@ struct Radau {
   // ignored, as the reference skips it): that keeps E2 defined on every path.
   __device__ __forceinline__ int decomp(Ctx& ctx) {
     const int ln = Grp<G>::lane();
-    const double g1 = rkGamma / H, g2r = rkAlpha / H, g2i = rkBeta / H;
+    const double iH = 1.0 / H;
+    const double g1 = quot(rkGamma, H, iH), g2r = quot(rkAlpha, H, iH), g2i = quot(rkBeta, H, iH);
     int info = 0, info2 = 0;
     if constexpr (Mech::kJacInLds) group_lds_sync();
     auto jac_at = [&](int q, int r, int j) -> double {
@@ -1695,8 +1779,27 @@ struct Radau {
     for (int q = 0; q < R; ++q)
       if (RW::valid(ln, q)) s += sc[q] * sc[q] * d[q] * d[q];
     s = Grp<G>::sum(s);
-    const double e = sqrt(s / (double)N);
+    const double e = sqrt(quot(s, (double)N, 1.0 / (double)N));
     return e == e ? fmax(e, 1e-10) : __builtin_inf();
+  }
+  // The root mean square of the three stages' norms (the Newton increment,
+  // radau2a.c:640-645): from the sums of squares under the norms' floor, with one
+  // root and one division instead of four each.
+  __device__ __forceinline__ double err_norm3(const double (&d1)[R], const double (&d2)[R], const double (&d3)[R]) const {
+    const int ln = Grp<G>::lane();
+    double s1 = 0.0, s2 = 0.0, s3 = 0.0;
+#pragma unroll
+    for (int q = 0; q < R; ++q)
+      if (RW::valid(ln, q)) {
+        const double w = sc[q] * sc[q];
+        s1 += w * d1[q] * d1[q];
+        s2 += w * d2[q] * d2[q];
+        s3 += w * d3[q] * d3[q];
+      }
+    Grp<G>::sum3(s1, s2, s3);
+    constexpr double floor_ = 1e-20 * N;
+    const double e = sqrt(quot(fmax(s1, floor_) + fmax(s2, floor_) + fmax(s3, floor_), 3.0 * N, 1.0 / (3.0 * N)));
+    return s1 + s2 + s3 == s1 + s2 + s3 ? e : __builtin_inf();  // (fmax drops a NaN)
   }
 
   // integrate() prologue, radau2a.c:521-564: a fresh start for every interval.
@@ -1808,12 +1911,13 @@ struct Radau {
         Z3[q] = CONT0[q] + x2 * (CONT1[q] + x3 * CONT2[q]);
       }
     }
+    const double iH = 1.0 / H;
     bool NewtonDone = false;
     double NewtonIncrementOld = 0.0;
     double Fac = 0.5;
     int NewtonIter = 0;
     double Theta = 0.0;
-    NewtonRate = step_pow(fmax(NewtonRate, kRoundoff), 0.8);
+    NewtonRate = pow_0p8(fmax(NewtonRate, kRoundoff));
 
 #pragma unroll 1
     for (; NewtonIter < kNewtonMaxit; NewtonIter++) {
@@ -1840,7 +1944,7 @@ struct Radau {
       {
 #pragma unroll
         for (int q = 0; q < R; ++q) {
-          const double x1 = DZ1[q] / H, x2 = DZ2[q] / H, x3 = DZ3[q] / H;
+          const double x1 = quot(DZ1[q], H, iH), x2 = quot(DZ2[q], H, iH), x3 = quot(DZ3[q], H, iH);
           DZ1[q] = rkTiAi00 * x1 + rkTiAi01 * x2 + rkTiAi02 * x3;
           DZ2[q] = rkTiAi10 * x1 + rkTiAi11 * x2 + rkTiAi12 * x3;
           DZ3[q] = rkTiAi20 * x1 + rkTiAi21 * x2 + rkTiAi22 * x3;
@@ -1858,10 +1962,7 @@ struct Radau {
         }
         cnt[CNT_NEWTON]++;
       }
-      const double d1 = err_norm(DZ1);
-      const double d2 = err_norm(DZ2);
-      const double d3 = err_norm(DZ3);
-      const double NewtonIncrement = sqrt((d1 * d1 + d2 * d2 + d3 * d3) / 3.0);
+      const double NewtonIncrement = err_norm3(DZ1, DZ2, DZ3);
       if (FirstStep && UseStart && NewtonIter == 0) {
         // A predicted start is kept only if its first Newton correction is
         // smaller than the corrected stages, i.e. than the zero start's
@@ -1869,8 +1970,7 @@ struct Radau {
         double W1[R], W2[R], W3[R];
 #pragma unroll
         for (int q = 0; q < R; ++q) { W1[q] = Z1[q] - DZ1[q]; W2[q] = Z2[q] - DZ2[q]; W3[q] = Z3[q] - DZ3[q]; }
-        const double w1 = err_norm(W1), w2 = err_norm(W2), w3 = err_norm(W3);
-        if (!(NewtonIncrement < sqrt((w1 * w1 + w2 * w2 + w3 * w3) / 3.0))) {
+        if (!(NewtonIncrement < err_norm3(W1, W2, W3))) {
           UseStart = false;
           StartFailed = true;
 #pragma unroll
@@ -1888,7 +1988,7 @@ struct Radau {
           break;
         }
         const double NewtonPredictedErr =
-            (NewtonIncrement * step_pow(Theta, (double)(kNewtonMaxit - NewtonIter - 1))) / (1.0 - Theta);
+            (NewtonIncrement * pow_int(Theta, kNewtonMaxit - NewtonIter - 1)) / (1.0 - Theta);
         if (NewtonPredictedErr >= kNewtonTol) {
           const double Qnewton = fmin(10.0, NewtonPredictedErr / kNewtonTol);
           Fac = 0.8 * step_pow(Qnewton, -1.0 / ((double)(kNewtonMaxit - NewtonIter)));
@@ -1944,7 +2044,7 @@ struct Radau {
     // rejected step with Err >= 1, solve again with f(t, y + x) + F2.
     double Err;
     {
-      const double HrkE1 = rkE1 / H, HrkE2 = rkE2 / H, HrkE3 = rkE3 / H;
+      const double HrkE1 = quot(rkE1, H, iH), HrkE2 = quot(rkE2, H, iH), HrkE3 = quot(rkE3, H, iH);
       double F2[R], Tm[R];
 #pragma unroll
       for (int q = 0; q < R; ++q) {
@@ -1966,14 +2066,14 @@ struct Radau {
         for (int q = 0; q < R; ++q) Tm[q] = F1[q] + F2[q];
       }
     }
-    Fac = step_pow(Err, (-1.0 / rkELO)) * (1.0 + 2 * kNewtonMaxit) / (NewtonIter + 1.0 + 2 * kNewtonMaxit);
+    Fac = inv_root4(Err) * (1.0 + 2 * kNewtonMaxit) / (NewtonIter + 1.0 + 2 * kNewtonMaxit);
     Fac = fmin(kFacMax, fmax(kFacMin, Fac));
     double Hnew = Fac * H;
     if (Err < 1.0) {
       cnt[CNT_ACCEPT]++;
       if (FirstStep && P.log.cap > 0) log_first_step(P.log, pr);
       if (!FirstStep) {  // Gustafsson, :676-685
-        double FacGus = kFacSafe * (H / Hacc) * step_pow(Err * Err / ErrOld, -0.25);
+        double FacGus = kFacSafe * (H / Hacc) * inv_root4(Err * Err / ErrOld);
         FacGus = fmin(kFacMax, fmax(kFacMin, FacGus));
         Fac = fmin(Fac, FacGus);
         Hnew = Fac * H;
@@ -1987,15 +2087,15 @@ struct Radau {
       for (int q = 0; q < R; ++q) y[q] += Z3[q];
       // RK_Make_Interpolate, :283-297
       {
-        constexpr double den = (rkC2 - rkC1) * (rkC1 - rkC0) * (rkC0 - rkC2);
+        constexpr double den = (rkC2 - rkC1) * (rkC1 - rkC0) * (rkC0 - rkC2), iden = 1.0 / den;
 #pragma unroll
         for (int q = 0; q < R; ++q) {
           const double z1 = Z1[q], z2 = Z2[q], z3 = Z3[q];
-          CONT0[q] = ((-rkC2 * rkC2 * rkC1 * z1 + z3 * rkC1 * rkC0 * rkC0 + rkC1 * rkC1 * rkC2 * z1 -
-                       rkC1 * rkC1 * rkC0 * z3 + rkC2 * rkC2 * rkC0 * z2 - z2 * rkC2 * rkC0 * rkC0) /
-                      den) - z3;
-          CONT1[q] = -(rkC0 * rkC0 * (z3 - z2) + rkC1 * rkC1 * (z1 - z3) + rkC2 * rkC2 * (z2 - z1)) / den;
-          CONT2[q] = (rkC0 * (z3 - z2) + rkC1 * (z1 - z3) + rkC2 * (z2 - z1)) / den;
+          CONT0[q] = quot(-rkC2 * rkC2 * rkC1 * z1 + z3 * rkC1 * rkC0 * rkC0 + rkC1 * rkC1 * rkC2 * z1 -
+                              rkC1 * rkC1 * rkC0 * z3 + rkC2 * rkC2 * rkC0 * z2 - z2 * rkC2 * rkC0 * rkC0,
+                          den, iden) - z3;
+          CONT1[q] = -quot(rkC0 * rkC0 * (z3 - z2) + rkC1 * rkC1 * (z1 - z3) + rkC2 * rkC2 * (z2 - z1), den, iden);
+          CONT2[q] = quot(rkC0 * (z3 - z2) + rkC1 * (z1 - z3) + rkC2 * (z2 - z1), den, iden);
         }
       }
 #pragma unroll
