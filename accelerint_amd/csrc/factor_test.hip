@@ -138,8 +138,8 @@ __global__ __launch_bounds__(64) void k_factor_test_16(int num, const double* __
 
 // Order 112: the memory-resident blocked LU of the large systems (MemLU, one
 // wave per matrix, factors in the workspace ws: MemLU<112, 2, double>::bytes()
-// per matrix), explicit interchanges as LAPACK; perm[k] = the original row
-// that ends at position k (the row chosen at step k).
+// per matrix); perm[k] = the original row that ends at position k (the row
+// chosen at step k).
 template <class T, bool CPLX>
 __global__ __launch_bounds__(64) void k_factor_test_mem(int num, const double* __restrict__ a_re,
                                                         const double* __restrict__ a_im,
@@ -157,7 +157,7 @@ __global__ __launch_bounds__(64) void k_factor_test_mem(int num, const double* _
   T* E1 = reinterpret_cast<T*>(ws + (size_t)c * MemLU<N, R, double>::bytes());
   T* E2r = E1 + MLU::kMat;
   T* E2i = E2r + MLU::kMat;
-  int* ipiv = reinterpret_cast<int*>(E1 + 3 * MLU::kMat);
+  int* perm = CPLX ? MLU::perm2(E1) : MLU::perm1(E1);
   T* Er = CPLX ? E2r : E1;
   const size_t base = (size_t)c * N * N;
 #pragma unroll
@@ -172,8 +172,8 @@ __global__ __launch_bounds__(64) void k_factor_test_mem(int num, const double* _
   }
   wave_vmem_sync();
   int info = 0;
-  if constexpr (CPLX) MLU::factor_cplx(E2r, E2i, ipiv, info);
-  else MLU::factor_real(E1, ipiv, info);
+  if constexpr (CPLX) MLU::factor_cplx(E2r, E2i, perm, MLU::tmp(E1), info);
+  else MLU::factor_real(E1, perm, MLU::tmp(E1), info);
 #pragma unroll
   for (int q = 0; q < R; ++q) {
     const int r = ln + 64 * q;
@@ -185,15 +185,7 @@ __global__ __launch_bounds__(64) void k_factor_test_mem(int num, const double* _
     }
   }
   if (ln == 0) {
-    int at[N];
-    for (int i = 0; i < N; ++i) at[i] = i;
-    for (int k = 0; k < N; ++k) {
-      const int p = ipiv[k];
-      const int t = at[k];
-      at[k] = at[p];
-      at[p] = t;
-      perm_out[(size_t)c * N + k] = at[k];
-    }
+    for (int k = 0; k < N; ++k) perm_out[(size_t)c * N + k] = perm[k];
     info_out[c] = info;
   }
   if (b_re) {  // uniform over the launch
@@ -204,8 +196,8 @@ __global__ __launch_bounds__(64) void k_factor_test_mem(int num, const double* _
       br[q] = r < N ? (T)b_re[(size_t)c * N + r] : T(0);
       bi[q] = (CPLX && r < N) ? (T)b_im[(size_t)c * N + r] : T(0);
     }
-    if constexpr (CPLX) MLU::solve_cplx(E2r, E2i, ipiv, br, bi);
-    else MLU::solve_real(E1, ipiv, br);
+    if constexpr (CPLX) MLU::solve_cplx(E2r, E2i, perm, br, bi);
+    else MLU::solve_real(E1, perm, br);
 #pragma unroll
     for (int q = 0; q < R; ++q) {
       const int r = ln + 64 * q;

@@ -5,22 +5,33 @@
 //
 // dgetrf / zgetrf semantics (the reference's RK_Decomp, radau2a.c:256-278,
 // through LAPACK): partial pivoting on the first maximum of |a| (real) or
-// |Re| + |Im| (complex), explicit row interchanges, blocked right-looking:
+// |Re| + |Im| (complex), blocked right-looking with implicit interchanges --
+// rows stay where they are, each records the LAPACK position it would hold --
+// until one gather at the end puts them in order:
 //   1. the panel of 16 columns is factorized in registers (each lane holds its
-//      rows' 16 panel entries; pivot search by group argmax, the pivot row
-//      broadcast through SGPRs);
-//   2. the panel's interchanges are applied to the columns outside it (dlaswp);
-//   3. the pivot rows' trailing part is solved against the panel's unit-lower
+//      rows' 16 panel entries; one-word pivot search, the pivot row broadcast
+//      through SGPRs);
+//   2. the pivot rows' trailing part is solved against the panel's unit-lower
 //      block (dtrsm), lanes over columns;
-//   4. the trailing matrix takes the rank-16 update A22 -= L21 U12 on MFMA
+//   3. the trailing matrix takes the rank-16 update A22 -= L21 U12 on MFMA
 //      (v_mfma_{f32,f64}_16x16x4: four K = 4 steps per 16 x 16 tile; complex:
-//      four real products per step).
+//      four real products per step) over all row tiles, the rows already
+//      eliminated with zero multipliers: L21 (so masked) and U12 are taken from
+//      copies laid out for the operands, all of a column tile's loads are in
+//      flight together and L21 stays in registers for the whole panel.
 // Within a wave, global stores made by one lane are read by other lanes only
 // after s_waitcnt vmcnt(0): the wave's vector memory traffic goes through its
 // CU's write-through L1, so that wait makes them visible on the same CU.
-// The solves (dgetrs / zgetrs, radau2a.c:404,417) apply the interchanges to the
-// right-hand side and substitute column by column, skipping zero entries as
-// reference BLAS does.
+// The solves (dgetrs / zgetrs, radau2a.c:404,417) gather the right-hand side
+// and substitute column by column, skipping zero entries as reference BLAS
+// does, with the next block of columns loaded while one is used.
+//
+// Bound by latency: a single wave, workspace in L2.  With explicit interchanges
+// (a panel's 16 composed by wave-uniform index work and applied column by
+// column, 64 cache lines an access) and two row tiles in flight, an FP64 pair
+// took 4.8M cycles and the two solves 0.23M and 0.27M; now 1.7M, 0.07M and 0.12M
+// (24 112-state conditions beside 2049 54-state and 8190 14-state ones, one step in
+// FP64: 361.6 -> 131.9 ms).
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -58,166 +69,167 @@ struct MemLU {
   static constexpr int NT = N / 16;
   static constexpr size_t kMat = (size_t)LD * N;  // elements of one matrix
   static_assert(N % 16 == 0 && N > 64 && N <= LD, "memory LU: N a multiple of 16 in (64, 64 R]");
-  // workspace: E1, E2r, E2i (T, kMat each), then ipiv1[N], ipiv2[N] (int)
-  __host__ __device__ static constexpr size_t bytes() { return 3 * kMat * sizeof(T) + 2 * (size_t)N * sizeof(int); }
+  // workspace: E1, E2r, E2i (T, kMat each), then perm1[N], perm2[N] (int: the
+  // original row in each position), then a factorization's temporaries: L21
+  // (16 columns of LD) and U12 (16 entries per column), real and imaginary
+  static constexpr size_t kTmpL = (size_t)16 * LD, kTmpU = (size_t)16 * N;
+  __host__ __device__ static constexpr size_t bytes() {
+    return (3 * kMat + 2 * (kTmpL + kTmpU)) * sizeof(T) + 2 * (size_t)N * sizeof(int);
+  }
+  __device__ __forceinline__ static int* perm1(T* ws) { return reinterpret_cast<int*>(ws + 3 * kMat); }
+  __device__ __forceinline__ static int* perm2(T* ws) { return perm1(ws) + N; }
+  __device__ __forceinline__ static T* tmp(T* ws) { return reinterpret_cast<T*>(perm1(ws) + 2 * N); }
 
-  __device__ __forceinline__ static int lane() { return (int)__lane_id(); }
+  // (pinned: with a lane index known to be constant the compiler computes every
+  // address of every phase once per kernel and keeps them in scratch)
+  __device__ __forceinline__ static int lane() {
+    int l = (int)__lane_id();
+    pin(l);
+    return l;
+  }
   // uniform broadcast of row r's value v (r runtime-uniform)
   __device__ __forceinline__ static T row_value(const T (&v)[R], int r) {
     return Grp<64>::bcast(sel<R>(v, r >> 6), r & 63);
   }
 
+  // Pivot of step c among the rows with position >= c: the row, wave-uniform.
+  // The leading 32 bits of the magnitudes decide (see wave_pivot); if no
+  // candidate compares (a NaN column) the row at position c stays, as idamax
+  // returns its first index when nothing compares greater.
+  __device__ __forceinline__ static int pivot(const T (&v)[R], const int (&pos)[R], int c) {
+    unsigned key[R], m = 0;
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      key[q] = pos[q] >= c && v[q] == v[q] ? mag_hi(v[q]) + 1u : 0u;
+      m = max_u(m, key[q]);
+    }
+    m = dpp_max_u<kDppXor1>(m);
+    m = dpp_max_u<kDppXor2>(m);
+    m = dpp_max_u<kDppHalfMirror>(m);
+    m = dpp_max_u<kDppMirror>(m);
+    int x = (int)m, y = (int)m;
+    swap_row_pairs(x, y);
+    x = y = (int)max_u((unsigned)x, (unsigned)y);
+    swap_halves(x, y);
+    m = (unsigned)__builtin_amdgcn_readfirstlane((int)max_u((unsigned)x, (unsigned)y));
+    unsigned long long cand[R];
+    int n = 0, row = 0;
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      cand[q] = __builtin_amdgcn_ballot_w64(m != 0 ? key[q] == m : pos[q] == c);
+      n += __builtin_popcountll(cand[q]);
+      row = cand[q] ? 64 * q + (int)__builtin_ctzll(cand[q]) : row;
+    }
+    if (__builtin_expect(n > 1, 0)) {
+      row = -1;
+      T bv = T(0);
+      int best = 0;
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        unsigned long long w = cand[q];
+        while (w) {
+          const int l = (int)__builtin_ctzll(w);
+          w &= w - 1;
+          const T vl = Grp<64>::bcast(v[q], l);
+          const int pl = __builtin_amdgcn_readlane(pos[q], l);
+          if (row < 0 || vl > bv || (vl == bv && pl < best)) {
+            bv = vl;
+            best = pl;
+            row = 64 * q + l;
+          }
+        }
+      }
+    }
+    return __builtin_amdgcn_readfirstlane(row);
+  }
+  __device__ __forceinline__ static int row_value(const int (&v)[R], int r) {
+    return Grp<64>::bcast_i(sel<R>(v, r >> 6), r & 63);
+  }
+  __device__ __forceinline__ static void init_pos(int (&pos)[R]) {
+#pragma unroll
+    for (int q = 0; q < R; ++q) pos[q] = (int)__lane_id() + 64 * q < N ? (int)__lane_id() + 64 * q : -1;
+  }
+  // position bookkeeping of one interchange: row p to position c
+  __device__ __forceinline__ static void take(int (&pos)[R], int p, int c) {
+    const int ppos = row_value(pos, p);
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      pos[q] = (int)__lane_id() + 64 * q == p ? c : (pos[q] == c ? ppos : pos[q]);
+      pin(pos[q]);
+    }
+  }
+
   // ---- real ------------------------------------------------------------------
-  __device__ static void panel_real(T* E, int* ipiv, int k, T (&pv)[R][16], int (&piv)[16], int& info) {
+  __device__ __forceinline__ static void panel_real(T* E, T* L, int k, T (&pv)[R][16], int (&pos)[R], int (&piv)[16],
+                                                    int& info) {
     const int ln = lane();
+#pragma unroll
+    for (int q = 0; q < R; ++q)
+#pragma unroll
+      for (int c = 0; c < 16; ++c) pv[q][c] = E[(size_t)(k + c) * LD + ln + 64 * q];  // rows up to LD are in the workspace
+#pragma unroll
+    for (int kk = 0; kk < 16; ++kk) {
+      const int c = k + kk;
+      T mag[R], col[R];
+#pragma unroll
+      for (int q = 0; q < R; ++q) mag[q] = fabs(pv[q][kk]);
+      const int p = pivot(mag, pos, c);
+      piv[kk] = p;
+      take(pos, p, c);
+#pragma unroll
+      for (int q = 0; q < R; ++q) col[q] = pv[q][kk];
+      const T pval = row_value(col, p);
+      const bool nz = !is_zero(pval);
+      info = !nz && info == 0 ? c + 1 : info;
+      const T rp = recip(pval);
+      const bool tiny = std::is_same<T, double>::value && fabs(pval) < min_normal<T>();
+      T l[R];
+#pragma unroll
+      for (int q = 0; q < R; ++q) {
+        T v = pv[q][kk] * rp;
+        if (__builtin_expect(tiny, 0)) v = pv[q][kk] / pval;
+        // (with a zero pivot the column's active part is zero: nothing to add)
+        const bool act = nz && pos[q] > c;
+        pv[q][kk] = act ? v : pv[q][kk];
+        l[q] = act ? -v : T(-0.0);
+        pin(pv[q][kk]);
+        pin(l[q]);
+      }
+#pragma unroll
+      for (int c2 = kk + 1; c2 < 16; ++c2) {
+#pragma unroll
+        for (int q = 0; q < R; ++q) col[q] = pv[q][c2];
+        const T u = row_value(col, p);
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+          pv[q][c2] = fma(l[q], u, pv[q][c2]);
+          pin(pv[q][c2]);
+        }
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
 #pragma unroll
     for (int q = 0; q < R; ++q) {
       const int r = ln + 64 * q;
 #pragma unroll
       for (int c = 0; c < 16; ++c) {
-        const T v = E[(size_t)(k + c) * LD + r];  // rows up to LD are in the workspace
-        pv[q][c] = (r >= k && r < N) ? v : T(0);
-      }
-    }
-#pragma unroll
-    for (int kk = 0; kk < 16; ++kk) {
-      const int c = k + kk;
-      T bv = T(-1);
-      int bkey = 0x7fffffff;
-#pragma unroll
-      for (int q = 0; q < R; ++q) {
-        const int r = ln + 64 * q;
-        const T v = fabs(pv[q][kk]);
-        const bool better = r >= c && r < N && (v > bv || (v == bv && r < bkey));
-        bv = better ? v : bv;
-        bkey = better ? r : bkey;
-      }
-      group_argmax<64>(bv, bkey);
-      // no candidate compares (a NaN column): keep row c, as idamax returns
-      // its first index when nothing compares greater; the pivot index then
-      // addresses memory only inside the matrix
-      const int pk = __builtin_amdgcn_readfirstlane(bkey);
-      const int p = (pk >= c && pk < N) ? pk : c;
-      piv[kk] = p;
-      // the pivot row's and row c's panel entries
-      T prow[16], crow[16];
-#pragma unroll
-      for (int c2 = 0; c2 < 16; ++c2) {
-        T col[R];
-#pragma unroll
-        for (int q = 0; q < R; ++q) col[q] = pv[q][c2];
-        prow[c2] = row_value(col, p);
-        crow[c2] = row_value(col, c);
-      }
-      const T pval = prow[kk];
-      const bool nz = pval != T(0);
-      if (!nz && info == 0) info = c + 1;
-      if (nz && p != c) {
-#pragma unroll
-        for (int q = 0; q < R; ++q) {
-          const int r = ln + 64 * q;
-#pragma unroll
-          for (int c2 = 0; c2 < 16; ++c2) pv[q][c2] = r == c ? prow[c2] : (r == p ? crow[c2] : pv[q][c2]);
-        }
-      }
-      // row c after the interchange is the pivot row (with a zero pivot the
-      // column below is zero: p == c and the update adds nothing)
-      const bool tiny = std::is_same<T, double>::value && fabs(pval) < min_normal<T>();
-      const T rp = recip(pval);
-#pragma unroll
-      for (int q = 0; q < R; ++q) {
-        const int r = ln + 64 * q;
-        const bool act = nz && r > c && r < N;
-        const T l = tiny ? pv[q][kk] / pval : pv[q][kk] * rp;
-        pv[q][kk] = act ? l : pv[q][kk];
-        const T lm = (r > c && r < N) ? pv[q][kk] : T(0);
-#pragma unroll
-        for (int c2 = kk + 1; c2 < 16; ++c2) pv[q][c2] = fma(-lm, prow[c2], pv[q][c2]);
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < R; ++q) {
-      const int r = ln + 64 * q;
-      if (r >= k && r < N) {
-#pragma unroll
-        for (int c = 0; c < 16; ++c) E[(size_t)(k + c) * LD + r] = pv[q][c];
-      }
-    }
-    if (ln == 0) {
-#pragma unroll
-      for (int kk = 0; kk < 16; ++kk) ipiv[k + kk] = piv[kk];
-    }
-  }
-
-  // The panel's 16 interchanges (rows k + kk and piv[kk] >= k + kk, in order)
-  // composed into one permutation of the rows they touch.  Slots 0..15 name
-  // rows k..k+15, slots 16..31 the pivot rows; a slot is canonical if no
-  // earlier slot names the same row.  After the interchanges, the row of
-  // canonical slot s holds what row who[s] held before.  Wave-uniform index
-  // work, written with selects only (no dynamically indexed arrays).
-  struct Moves {
-    int row[32], who[32];
-    bool moved[32];
-  };
-  __device__ static void compose(int k, const int (&piv)[16], Moves& mv) {
-    int canon[32];
-#pragma unroll
-    for (int s = 0; s < 16; ++s) {
-      mv.row[s] = k + s;
-      mv.row[16 + s] = piv[s];
-    }
-#pragma unroll
-    for (int s = 0; s < 32; ++s) {
-      canon[s] = s;
-#pragma unroll
-      for (int s2 = s - 1; s2 >= 0; --s2) canon[s] = mv.row[s2] == mv.row[s] ? s2 : canon[s];
-      mv.who[s] = mv.row[s];
-    }
-#pragma unroll
-    for (int kk = 0; kk < 16; ++kk) {
-      const int cp = canon[16 + kk];  // row k + kk is slot kk, canonical
-      const int t = mv.who[kk];
-      int w = mv.who[0];
-#pragma unroll
-      for (int s = 1; s < 32; ++s) w = cp == s ? mv.who[s] : w;
-      mv.who[kk] = w;
-#pragma unroll
-      for (int s = 0; s < 32; ++s) mv.who[s] = cp == s ? t : mv.who[s];
-    }
-#pragma unroll
-    for (int s = 0; s < 32; ++s) mv.moved[s] = canon[s] == s && mv.who[s] != mv.row[s];
-  }
-
-  // dlaswp of the panel's 16 interchanges on the columns outside it (lanes
-  // over columns: every access of a column is made by the same lane): the
-  // moved entries of a column are all loaded, then all stored
-  __device__ static void swaps(T* E, int k, const Moves& mv) {
-    const int ln = lane();
-#pragma unroll
-    for (int m = 0; m < (N + 63) / 64; ++m) {
-      const int j = ln + 64 * m;
-      if (j < N && (j < k || j >= k + 16)) {
-        T* col = E + (size_t)j * LD;
-        T v[32];
-#pragma unroll
-        for (int s = 0; s < 32; ++s) v[s] = col[mv.who[s]];
-#pragma unroll
-        for (int s = 0; s < 32; ++s)
-          if (mv.moved[s]) col[mv.row[s]] = v[s];
+        E[(size_t)(k + c) * LD + r] = pv[q][c];
+        L[(size_t)c * LD + r] = pos[q] >= k + 16 ? -pv[q][c] : T(0);
       }
     }
   }
 
-  // U12 = L11^-1 A12 on the 16 pivot rows, columns k+16 .. N-1 (lanes over columns)
-  __device__ static void trsm_real(T* E, int k, const T (&pv)[R][16]) {
+  // U12 = L11^-1 A12 on the 16 pivot rows, columns k+16 .. N-1 (lanes over
+  // columns), into the matrix and, 16 entries per column, into U
+  __device__ __forceinline__ static void trsm_real(T* E, T* U, int k, const T (&pv)[R][16], const int (&piv)[16]) {
     const int ln = lane();
     constexpr int M = (N + 63) / 64;
     T u[M][16];
 #pragma unroll
     for (int m = 0; m < M; ++m) {
-      const int j = k + 16 + ln + 64 * m;
+      const int j = min(k + 16 + ln + 64 * m, N - 1);
 #pragma unroll
-      for (int i = 0; i < 16; ++i) u[m][i] = j < N ? E[(size_t)j * LD + k + i] : T(0);
+      for (int i = 0; i < 16; ++i) u[m][i] = E[(size_t)j * LD + piv[i]];
     }
 #pragma unroll
     for (int i = 1; i < 16; ++i) {
@@ -226,7 +238,7 @@ struct MemLU {
         T col[R];
 #pragma unroll
         for (int q = 0; q < R; ++q) col[q] = pv[q][mm];
-        const T lim = row_value(col, k + i);  // L(k+i, k+mm)
+        const T lim = row_value(col, piv[i]);  // L(k+i, k+mm)
 #pragma unroll
         for (int m = 0; m < M; ++m) u[m][i] = fma(-lim, u[m][mm], u[m][i]);
       }
@@ -236,209 +248,212 @@ struct MemLU {
       const int j = k + 16 + ln + 64 * m;
       if (j < N) {
 #pragma unroll
-        for (int i = 1; i < 16; ++i) E[(size_t)j * LD + k + i] = u[m][i];
+        for (int i = 0; i < 16; ++i) {
+          U[(size_t)j * 16 + i] = u[m][i];
+          if (i > 0) E[(size_t)j * LD + piv[i]] = u[m][i];
+        }
       }
     }
   }
 
-  // A22 -= L21 U12 (rows and columns k+16 .. N-1) on MFMA
-  __device__ static void update_real(T* E, int k) {
+  // A22 -= L21 U12 (columns k+16 .. N-1, all rows) on MFMA
+  __device__ __forceinline__ static void update_real(T* E, const T* L, const T* U, int k) {
     const int ln = lane(), lr = ln & 15, lq = ln >> 4;
-    const int t0 = k / 16 + 1;
+    T a[NT][4];
+#pragma unroll
+    for (int rt = 0; rt < NT; ++rt)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) a[rt][t] = L[(size_t)(4 * t + lq) * LD + rt * 16 + lr];
 #pragma unroll 1
-    for (int cb = t0; cb < NT; ++cb) {
-      const T* ccol = E + (size_t)(cb * 16 + lr) * LD;
+    for (int cb = k / 16 + 1; cb < NT; ++cb) {
+      T* ccol = E + (size_t)(cb * 16 + lr) * LD;
       T b[4];
 #pragma unroll
-      for (int t = 0; t < 4; ++t) b[t] = ccol[k + 4 * t + lq];
-      // two row tiles per pass (the second a repeat of the first, not
-      // stored, when the count is odd): their loads overlap
-#pragma unroll 1
-      for (int rb = t0; rb < NT; rb += 2) {
-        const bool two = rb + 1 < NT;
-        const int rbs[2] = {rb, two ? rb + 1 : rb};
-        T a[2][4];
-        mfma_vec<T> acc[2];
-        T* d[2];
+      for (int t = 0; t < 4; ++t) b[t] = U[(size_t)(cb * 16 + lr) * 16 + 4 * t + lq];
+      mfma_vec<T> acc[NT];
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
+      for (int rt = 0; rt < NT; ++rt)
 #pragma unroll
-          for (int t = 0; t < 4; ++t) a[u][t] = -E[(size_t)(k + 4 * t + lq) * LD + rbs[u] * 16 + lr];
-          d[u] = E + (size_t)(cb * 16 + lr) * LD + rbs[u] * 16;
+        for (int i = 0; i < 4; ++i) acc[rt][i] = ccol[rt * 16 + d_row<T>(lq, i)];
 #pragma unroll
-          for (int i = 0; i < 4; ++i) acc[u][i] = d[u][d_row<T>(lq, i)];
-        }
+      for (int t = 0; t < 4; ++t)
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
+        for (int rt = 0; rt < NT; ++rt) acc[rt] = mfma16x16x4(a[rt][t], b[t], acc[rt]);
 #pragma unroll
-          for (int t = 0; t < 4; ++t) acc[u] = mfma16x16x4(a[u][t], b[t], acc[u]);
-        }
+      for (int rt = 0; rt < NT; ++rt)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) d[0][d_row<T>(lq, i)] = acc[0][i];
-        if (two) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) d[1][d_row<T>(lq, i)] = acc[1][i];
-        }
-      }
+        for (int i = 0; i < 4; ++i) ccol[rt * 16 + d_row<T>(lq, i)] = acc[rt][i];
     }
   }
 
-  __device__ static void factor_real(T* E, int* ipiv, int& info) {
+  // rows into their positions (perm: the original row of every position)
+  __device__ __forceinline__ static void order_rows(T* E, const int* perm) {
+    const int ln = lane();
+    int src[R];
+#pragma unroll
+    for (int q = 0; q < R; ++q) src[q] = perm[min(ln + 64 * q, N - 1)];
+#pragma unroll 1
+    for (int j0 = 0; j0 < N; j0 += 16) {
+      T v[R][16];
+#pragma unroll
+      for (int q = 0; q < R; ++q)
+#pragma unroll
+        for (int c = 0; c < 16; ++c) v[q][c] = E[(size_t)(j0 + c) * LD + src[q]];
+      wave_vmem_sync();  // every lane has read before any writes
+#pragma unroll
+      for (int q = 0; q < R; ++q)
+#pragma unroll
+        for (int c = 0; c < 16; ++c) E[(size_t)(j0 + c) * LD + ln + 64 * q] = v[q][c];
+    }
+  }
+
+  __device__ __forceinline__ static void store_piv(int* perm, int k, const int (&piv)[16]) {
+    if (lane() == 0) {
+#pragma unroll
+      for (int kk = 0; kk < 16; ++kk) perm[k + kk] = piv[kk];
+    }
+  }
+
+  __device__ static void factor_real(T* E, int* perm, T* tmp, int& info) {
+    T *L = tmp, *U = tmp + kTmpL;
+    int pos[R];
+    init_pos(pos);
     info = 0;
 #pragma unroll 1
     for (int k = 0; k < N; k += 16) {
       T pv[R][16];
       int piv[16];
-      panel_real(E, ipiv, k, pv, piv, info);
-      Moves mv;
-      compose(k, piv, mv);
-      swaps(E, k, mv);
+      panel_real(E, L, k, pv, pos, piv, info);
+      store_piv(perm, k, piv);
       if (k + 16 < N) {
         wave_vmem_sync();
-        trsm_real(E, k, pv);
+        trsm_real(E, U, k, pv, piv);
         wave_vmem_sync();
-        update_real(E, k);
+        update_real(E, L, U, k);
       }
       wave_vmem_sync();
     }
+    order_rows(E, perm);
+    wave_vmem_sync();
   }
 
   // ---- complex ---------------------------------------------------------------
-  __device__ static void panel_cplx(T* Er, T* Ei, int* ipiv, int k, T (&pr)[R][16], T (&pi)[R][16],
-                                    int (&piv)[16], int& info) {
+  __device__ __forceinline__ static void panel_cplx(T* Er, T* Ei, T* Lr, T* Li, int k, T (&pr)[R][16], T (&pi)[R][16],
+                                                    int (&pos)[R], int (&piv)[16], int& info) {
     const int ln = lane();
 #pragma unroll
-    for (int q = 0; q < R; ++q) {
-      const int r = ln + 64 * q;
+    for (int q = 0; q < R; ++q)
 #pragma unroll
       for (int c = 0; c < 16; ++c) {
-        const bool in = r >= k && r < N;
-        const T vr = Er[(size_t)(k + c) * LD + r], vi = Ei[(size_t)(k + c) * LD + r];
-        pr[q][c] = in ? vr : T(0);
-        pi[q][c] = in ? vi : T(0);
+        pr[q][c] = Er[(size_t)(k + c) * LD + ln + 64 * q];
+        pi[q][c] = Ei[(size_t)(k + c) * LD + ln + 64 * q];
       }
-    }
 #pragma unroll
     for (int kk = 0; kk < 16; ++kk) {
       const int c = k + kk;
-      T bv = T(-1);
-      int bkey = 0x7fffffff;
+      T mag[R], cr[R], ci[R];
+#pragma unroll
+      for (int q = 0; q < R; ++q) mag[q] = fabs(pr[q][kk]) + fabs(pi[q][kk]);
+      const int p = pivot(mag, pos, c);
+      piv[kk] = p;
+      take(pos, p, c);
 #pragma unroll
       for (int q = 0; q < R; ++q) {
-        const int r = ln + 64 * q;
-        const T v = fabs(pr[q][kk]) + fabs(pi[q][kk]);
-        const bool better = r >= c && r < N && (v > bv || (v == bv && r < bkey));
-        bv = better ? v : bv;
-        bkey = better ? r : bkey;
+        cr[q] = pr[q][kk];
+        ci[q] = pi[q][kk];
       }
-      group_argmax<64>(bv, bkey);
-      // no candidate compares (a NaN column): keep row c, as idamax returns
-      // its first index when nothing compares greater; the pivot index then
-      // addresses memory only inside the matrix
-      const int pk = __builtin_amdgcn_readfirstlane(bkey);
-      const int p = (pk >= c && pk < N) ? pk : c;
-      piv[kk] = p;
-      T prr[16], pri[16], crr[16], cri[16];
-#pragma unroll
-      for (int c2 = 0; c2 < 16; ++c2) {
-        T colr[R], coli[R];
-#pragma unroll
-        for (int q = 0; q < R; ++q) { colr[q] = pr[q][c2]; coli[q] = pi[q][c2]; }
-        prr[c2] = row_value(colr, p);
-        pri[c2] = row_value(coli, p);
-        crr[c2] = row_value(colr, c);
-        cri[c2] = row_value(coli, c);
-      }
-      const T vr = prr[kk], vi = pri[kk];
-      const bool nz = vr != T(0) || vi != T(0);
-      if (!nz && info == 0) info = c + 1;
-      if (nz && p != c) {
-#pragma unroll
-        for (int q = 0; q < R; ++q) {
-          const int r = ln + 64 * q;
-#pragma unroll
-          for (int c2 = 0; c2 < 16; ++c2) {
-            pr[q][c2] = r == c ? prr[c2] : (r == p ? crr[c2] : pr[q][c2]);
-            pi[q][c2] = r == c ? pri[c2] : (r == p ? cri[c2] : pi[q][c2]);
-          }
-        }
-      }
+      const T vr = row_value(cr, p), vi = row_value(ci, p);
+      const bool nz = !(is_zero(vr) && is_zero(vi));
+      info = !nz && info == 0 ? c + 1 : info;
       T rr, ri;
       crecip(vr, vi, rr, ri);
+      T lr[R], li[R];
 #pragma unroll
       for (int q = 0; q < R; ++q) {
-        const int r = ln + 64 * q;
-        const bool act = nz && r > c && r < N;
         const T xr = pr[q][kk], xi = pi[q][kk];
         const T sr = xr * rr - xi * ri, si = xr * ri + xi * rr;
+        const bool act = nz && pos[q] > c;
         pr[q][kk] = act ? sr : xr;
         pi[q][kk] = act ? si : xi;
-        const bool below = r > c && r < N;
-        const T lr = below ? pr[q][kk] : T(0), li = below ? pi[q][kk] : T(0);
+        lr[q] = act ? sr : T(0);
+        li[q] = act ? si : T(0);
+        pin(pr[q][kk]);
+        pin(pi[q][kk]);
+        pin(lr[q]);
+        pin(li[q]);
+      }
 #pragma unroll
-        for (int c2 = kk + 1; c2 < 16; ++c2) {
-          pr[q][c2] = fma(-lr, prr[c2], pr[q][c2]);
-          pr[q][c2] = fma(li, pri[c2], pr[q][c2]);
-          pi[q][c2] = fma(-lr, pri[c2], pi[q][c2]);
-          pi[q][c2] = fma(-li, prr[c2], pi[q][c2]);
+      for (int c2 = kk + 1; c2 < 16; ++c2) {
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+          cr[q] = pr[q][c2];
+          ci[q] = pi[q][c2];
+        }
+        const T ur = row_value(cr, p), ui = row_value(ci, p);
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+          pr[q][c2] = fma(li[q], ui, fma(-lr[q], ur, pr[q][c2]));
+          pi[q][c2] = fma(-li[q], ur, fma(-lr[q], ui, pi[q][c2]));
+          pin(pr[q][c2]);
+          pin(pi[q][c2]);
         }
       }
+      __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
     for (int q = 0; q < R; ++q) {
       const int r = ln + 64 * q;
-      if (r >= k && r < N) {
+      const bool below = pos[q] >= k + 16;
 #pragma unroll
-        for (int c = 0; c < 16; ++c) {
-          Er[(size_t)(k + c) * LD + r] = pr[q][c];
-          Ei[(size_t)(k + c) * LD + r] = pi[q][c];
-        }
+      for (int c = 0; c < 16; ++c) {
+        Er[(size_t)(k + c) * LD + r] = pr[q][c];
+        Ei[(size_t)(k + c) * LD + r] = pi[q][c];
+        Lr[(size_t)c * LD + r] = below ? pr[q][c] : T(0);
+        Li[(size_t)c * LD + r] = below ? pi[q][c] : T(0);
       }
-    }
-    if (ln == 0) {
-#pragma unroll
-      for (int kk = 0; kk < 16; ++kk) ipiv[k + kk] = piv[kk];
     }
   }
 
-  __device__ static void trsm_cplx(T* Er, T* Ei, int k, const T (&pr)[R][16], const T (&pi)[R][16]) {
+  __device__ __forceinline__ static void trsm_cplx(T* Er, T* Ei, T* Ur, T* Ui, int k, const T (&pr)[R][16],
+                                                   const T (&pi)[R][16], const int (&piv)[16]) {
     const int ln = lane();
     constexpr int M = (N + 63) / 64;
-    T ur[M][16], ui[M][16];
-#pragma unroll
+#pragma unroll 1
     for (int m = 0; m < M; ++m) {
-      const int j = k + 16 + ln + 64 * m;
+      if (k + 16 + 64 * m >= N) break;
+      const int j = k + 16 + ln + 64 * m, jj = min(j, N - 1);
+      T ur[16], ui[16];
 #pragma unroll
       for (int i = 0; i < 16; ++i) {
-        ur[m][i] = j < N ? Er[(size_t)j * LD + k + i] : T(0);
-        ui[m][i] = j < N ? Ei[(size_t)j * LD + k + i] : T(0);
+        ur[i] = Er[(size_t)jj * LD + piv[i]];
+        ui[i] = Ei[(size_t)jj * LD + piv[i]];
       }
-    }
 #pragma unroll
-    for (int i = 1; i < 16; ++i) {
+      for (int i = 1; i < 16; ++i) {
 #pragma unroll
-      for (int mm = 0; mm < i; ++mm) {
-        T cr[R], ci[R];
+        for (int mm = 0; mm < i; ++mm) {
+          T cr[R], ci[R];
 #pragma unroll
-        for (int q = 0; q < R; ++q) { cr[q] = pr[q][mm]; ci[q] = pi[q][mm]; }
-        const T lr = row_value(cr, k + i), li = row_value(ci, k + i);
-#pragma unroll
-        for (int m = 0; m < M; ++m) {
-          ur[m][i] = fma(-lr, ur[m][mm], ur[m][i]);
-          ur[m][i] = fma(li, ui[m][mm], ur[m][i]);
-          ui[m][i] = fma(-lr, ui[m][mm], ui[m][i]);
-          ui[m][i] = fma(-li, ur[m][mm], ui[m][i]);
+          for (int q = 0; q < R; ++q) {
+            cr[q] = pr[q][mm];
+            ci[q] = pi[q][mm];
+          }
+          const T lr = row_value(cr, piv[i]), li = row_value(ci, piv[i]);
+          ur[i] = fma(-lr, ur[mm], ur[i]);
+          ur[i] = fma(li, ui[mm], ur[i]);
+          ui[i] = fma(-lr, ui[mm], ui[i]);
+          ui[i] = fma(-li, ur[mm], ui[i]);
         }
       }
-    }
-#pragma unroll
-    for (int m = 0; m < M; ++m) {
-      const int j = k + 16 + ln + 64 * m;
       if (j < N) {
 #pragma unroll
-        for (int i = 1; i < 16; ++i) {
-          Er[(size_t)j * LD + k + i] = ur[m][i];
-          Ei[(size_t)j * LD + k + i] = ui[m][i];
+        for (int i = 0; i < 16; ++i) {
+          Ur[(size_t)j * 16 + i] = ur[i];
+          Ui[(size_t)j * 16 + i] = ui[i];
+          if (i > 0) {
+            Er[(size_t)j * LD + piv[i]] = ur[i];
+            Ei[(size_t)j * LD + piv[i]] = ui[i];
+          }
         }
       }
     }
@@ -446,200 +461,237 @@ struct MemLU {
 
   // (Dr + i Di) -= (Lr + i Li)(Ur + i Ui) on MFMA: Dr += (-Lr) Ur + Li Ui,
   // Di += (-Lr) Ui + (-Li) Ur
-  __device__ static void update_cplx(T* Er, T* Ei, int k) {
+  __device__ __forceinline__ static void update_cplx(T* Er, T* Ei, const T* Lr, const T* Li, const T* Ur, const T* Ui,
+                                                     int k) {
     const int ln = lane(), lr = ln & 15, lq = ln >> 4;
-    const int t0 = k / 16 + 1;
+    T ar[NT][4], ai[NT][4];
+#pragma unroll
+    for (int rt = 0; rt < NT; ++rt)
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        const size_t a = (size_t)(4 * t + lq) * LD + rt * 16 + lr;
+        ar[rt][t] = Lr[a];
+        ai[rt][t] = Li[a];
+      }
 #pragma unroll 1
-    for (int cb = t0; cb < NT; ++cb) {
+    for (int cb = k / 16 + 1; cb < NT; ++cb) {
       const size_t cc = (size_t)(cb * 16 + lr) * LD;
       T br[4], bi[4];
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
-        br[t] = Er[cc + k + 4 * t + lq];
-        bi[t] = Ei[cc + k + 4 * t + lq];
+        br[t] = Ur[(size_t)(cb * 16 + lr) * 16 + 4 * t + lq];
+        bi[t] = Ui[(size_t)(cb * 16 + lr) * 16 + 4 * t + lq];
       }
-#pragma unroll 1
-      for (int rb = t0; rb < NT; rb += 2) {
-        const bool two = rb + 1 < NT;
-        const int rbs[2] = {rb, two ? rb + 1 : rb};
-        T ar[2][4], ai[2][4];
-        mfma_vec<T> xr[2], xi[2];
-        T *dr[2], *di[2];
+      mfma_vec<T> xr[NT], xi[NT];
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-#pragma unroll
-          for (int t = 0; t < 4; ++t) {
-            const size_t a = (size_t)(k + 4 * t + lq) * LD + rbs[u] * 16 + lr;
-            ar[u][t] = Er[a];
-            ai[u][t] = Ei[a];
-          }
-          dr[u] = Er + cc + rbs[u] * 16;
-          di[u] = Ei + cc + rbs[u] * 16;
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            xr[u][i] = dr[u][d_row<T>(lq, i)];
-            xi[u][i] = di[u][d_row<T>(lq, i)];
-          }
-        }
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-#pragma unroll
-          for (int t = 0; t < 4; ++t) {
-            xr[u] = mfma16x16x4(-ar[u][t], br[t], xr[u]);
-            xr[u] = mfma16x16x4(ai[u][t], bi[t], xr[u]);
-            xi[u] = mfma16x16x4(-ar[u][t], bi[t], xi[u]);
-            xi[u] = mfma16x16x4(-ai[u][t], br[t], xi[u]);
-          }
-        }
+      for (int rt = 0; rt < NT; ++rt)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          dr[0][d_row<T>(lq, i)] = xr[0][i];
-          di[0][d_row<T>(lq, i)] = xi[0][i];
+          xr[rt][i] = Er[cc + rt * 16 + d_row<T>(lq, i)];
+          xi[rt][i] = Ei[cc + rt * 16 + d_row<T>(lq, i)];
         }
-        if (two) {
 #pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            dr[1][d_row<T>(lq, i)] = xr[1][i];
-            di[1][d_row<T>(lq, i)] = xi[1][i];
-          }
+      for (int t = 0; t < 4; ++t) {
+#pragma unroll
+        for (int rt = 0; rt < NT; ++rt) {
+          xr[rt] = mfma16x16x4(-ar[rt][t], br[t], xr[rt]);
+          xi[rt] = mfma16x16x4(-ar[rt][t], bi[t], xi[rt]);
+        }
+#pragma unroll
+        for (int rt = 0; rt < NT; ++rt) {
+          xr[rt] = mfma16x16x4(ai[rt][t], bi[t], xr[rt]);
+          xi[rt] = mfma16x16x4(-ai[rt][t], br[t], xi[rt]);
         }
       }
+#pragma unroll
+      for (int rt = 0; rt < NT; ++rt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          Er[cc + rt * 16 + d_row<T>(lq, i)] = xr[rt][i];
+          Ei[cc + rt * 16 + d_row<T>(lq, i)] = xi[rt][i];
+        }
     }
   }
 
-  __device__ static void factor_cplx(T* Er, T* Ei, int* ipiv, int& info) {
+  __device__ static void factor_cplx(T* Er, T* Ei, int* perm, T* tmp, int& info) {
+    T *Lr = tmp, *Li = Lr + kTmpL, *Ur = Li + kTmpL, *Ui = Ur + kTmpU;
+    int pos[R];
+    init_pos(pos);
     info = 0;
 #pragma unroll 1
     for (int k = 0; k < N; k += 16) {
       T pr[R][16], pi[R][16];
       int piv[16];
-      panel_cplx(Er, Ei, ipiv, k, pr, pi, piv, info);
-      Moves mv;
-      compose(k, piv, mv);
-      swaps(Er, k, mv);
-      swaps(Ei, k, mv);
+      panel_cplx(Er, Ei, Lr, Li, k, pr, pi, pos, piv, info);
+      store_piv(perm, k, piv);
       if (k + 16 < N) {
         wave_vmem_sync();
-        trsm_cplx(Er, Ei, k, pr, pi);
+        trsm_cplx(Er, Ei, Ur, Ui, k, pr, pi, piv);
         wave_vmem_sync();
-        update_cplx(Er, Ei, k);
+        update_cplx(Er, Ei, Lr, Li, Ur, Ui, k);
       }
       wave_vmem_sync();
     }
+    order_rows(Er, perm);
+    order_rows(Ei, perm);
+    wave_vmem_sync();
   }
 
   // ---- solves (nrhs = 1; b[q] = component of row lane + 64 q) ---------------
   // Every factor entry is loaded unconditionally (rows up to LD are in the
-  // workspace) and the update is selected, so the loads of the next columns
-  // are in flight while a column's update waits for its broadcast; a zero
+  // workspace) and the update is selected, so the next block of columns is in
+  // flight while a block's columns wait for each other's broadcasts; a zero
   // right-hand-side entry skips its column, as reference BLAS does.
-  __device__ static void laswp(const int* ipiv, T (&b)[R]) {
+  __device__ __forceinline__ static void gather(const int* perm, T (&b)[R]) {
     const int ln = lane();
+    T v[R];
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      const int src = perm[min(ln + 64 * q, N - 1)];
+      v[q] = __shfl(b[0], src & 63);
+#pragma unroll
+      for (int p = 1; p < R; ++p) {
+        const T w = __shfl(b[p], src & 63);
+        v[q] = (src >> 6) == p ? w : v[q];
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < R; ++q) b[q] = v[q];
+  }
+  template <int B>
+  __device__ __forceinline__ static void columns(const T* E, int k0, T (&l)[R][B]) {
+    const int ln = lane();
+#pragma unroll
+    for (int q = 0; q < R; ++q)
+#pragma unroll
+      for (int i = 0; i < B; ++i) l[q][i] = E[(size_t)(k0 + i) * LD + ln + 64 * q];
+  }
+
+  __device__ static void solve_real(const T* E, const int* perm, T (&b)[R]) {
+    constexpr int B = 16;
+    const int ln = lane();
+    T l[R][B], nx[R][B];
+    columns<B>(E, 0, nx);
+    gather(perm, b);
 #pragma unroll 1
-    for (int k0 = 0; k0 < N; k0 += 16) {
-      int p16[16];
+    for (int k0 = 0; k0 < N; k0 += B) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) p16[i] = __builtin_amdgcn_readfirstlane(ipiv[k0 + i]);
+      for (int q = 0; q < R; ++q)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int k = k0 + i, p = p16[i];
-        if (p != k) {
-          const T vk = row_value(b, k), vp = row_value(b, p);
+        for (int i = 0; i < B; ++i) l[q][i] = nx[q][i];
+      columns<B>(E, k0 + B < N ? k0 + B : N - B, nx);  // (at the end: the first block of the way back)
 #pragma unroll
-          for (int q = 0; q < R; ++q) {
-            const int r = ln + 64 * q;
-            b[q] = r == k ? vp : (r == p ? vk : b[q]);
-          }
+      for (int i = 0; i < B; ++i) {
+        const int k = k0 + i;
+        const T yk = row_value(b, k);
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+          const int r = ln + 64 * q;
+          const T nb = fma(-l[q][i], yk, b[q]);
+          b[q] = (yk != T(0) && r > k && r < N) ? nb : b[q];
+        }
+      }
+    }
+#pragma unroll 1
+    for (int k0 = N - B; k0 >= 0; k0 -= B) {
+#pragma unroll
+      for (int q = 0; q < R; ++q)
+#pragma unroll
+        for (int i = 0; i < B; ++i) l[q][i] = nx[q][i];
+      if (k0 > 0) columns<B>(E, k0 - B, nx);
+#pragma unroll
+      for (int i = B - 1; i >= 0; --i) {
+        const int k = k0 + i;
+        T col[R];
+#pragma unroll
+        for (int q = 0; q < R; ++q) col[q] = l[q][i];
+        const T bk = row_value(b, k);
+        const T xk = bk / row_value(col, k);
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+          const int r = ln + 64 * q;
+          const T nb = fma(-col[q], xk, b[q]);
+          b[q] = bk != T(0) ? (r < k ? nb : (r == k ? xk : b[q])) : b[q];
         }
       }
     }
   }
 
-  __device__ static void solve_real(const T* E, const int* ipiv, T (&b)[R]) {
+  __device__ static void solve_cplx(const T* Er, const T* Ei, const int* perm, T (&br)[R], T (&bi)[R]) {
+    constexpr int B = 8;
     const int ln = lane();
-    laswp(ipiv, b);
-#pragma unroll 8
-    for (int k = 0; k < N; ++k) {
-      const T yk = row_value(b, k);
-#pragma unroll
-      for (int q = 0; q < R; ++q) {
-        const int r = ln + 64 * q;
-        const T l = E[(size_t)k * LD + r];
-        const T nb = fma(-l, yk, b[q]);
-        b[q] = (yk != T(0) && r > k && r < N) ? nb : b[q];
-      }
-    }
-#pragma unroll 8
-    for (int k = N - 1; k >= 0; --k) {
-      const T bk = row_value(b, k);
-      const T xk = bk / E[(size_t)k * LD + k];
-#pragma unroll
-      for (int q = 0; q < R; ++q) {
-        const int r = ln + 64 * q;
-        const T u = E[(size_t)k * LD + r];
-        const T nb = fma(-u, xk, b[q]);
-        b[q] = bk != T(0) ? (r < k ? nb : (r == k ? xk : b[q])) : b[q];
-      }
-    }
-  }
-
-  __device__ static void solve_cplx(const T* Er, const T* Ei, const int* ipiv, T (&br)[R], T (&bi)[R]) {
-    const int ln = lane();
+    T lr[R][B], li[R][B], nr_[R][B], ni_[R][B];
+    columns<B>(Er, 0, nr_);
+    columns<B>(Ei, 0, ni_);
+    gather(perm, br);
+    gather(perm, bi);
 #pragma unroll 1
-    for (int k0 = 0; k0 < N; k0 += 16) {
-      int p16[16];
+    for (int k0 = 0; k0 < N; k0 += B) {
 #pragma unroll
-      for (int i = 0; i < 16; ++i) p16[i] = __builtin_amdgcn_readfirstlane(ipiv[k0 + i]);
+      for (int q = 0; q < R; ++q)
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int k = k0 + i, p = p16[i];
-        if (p != k) {
-          const T vkr = row_value(br, k), vpr = row_value(br, p);
-          const T vki = row_value(bi, k), vpi = row_value(bi, p);
+        for (int i = 0; i < B; ++i) {
+          lr[q][i] = nr_[q][i];
+          li[q][i] = ni_[q][i];
+        }
+      const int kn = k0 + B < N ? k0 + B : N - B;
+      columns<B>(Er, kn, nr_);
+      columns<B>(Ei, kn, ni_);
 #pragma unroll
-          for (int q = 0; q < R; ++q) {
-            const int r = ln + 64 * q;
-            br[q] = r == k ? vpr : (r == p ? vkr : br[q]);
-            bi[q] = r == k ? vpi : (r == p ? vki : bi[q]);
-          }
+      for (int i = 0; i < B; ++i) {
+        const int k = k0 + i;
+        const T yr = row_value(br, k), yi = row_value(bi, k);
+        const bool go = yr != T(0) || yi != T(0);
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+          const int r = ln + 64 * q;
+          T nr = fma(-lr[q][i], yr, br[q]);
+          nr = fma(li[q][i], yi, nr);
+          T ni = fma(-lr[q][i], yi, bi[q]);
+          ni = fma(-li[q][i], yr, ni);
+          const bool act = go && r > k && r < N;
+          br[q] = act ? nr : br[q];
+          bi[q] = act ? ni : bi[q];
         }
       }
     }
-#pragma unroll 8
-    for (int k = 0; k < N; ++k) {
-      const T yr = row_value(br, k), yi = row_value(bi, k);
-      const bool go = yr != T(0) || yi != T(0);
+#pragma unroll 1
+    for (int k0 = N - B; k0 >= 0; k0 -= B) {
 #pragma unroll
-      for (int q = 0; q < R; ++q) {
-        const int r = ln + 64 * q;
-        const T lr = Er[(size_t)k * LD + r], li = Ei[(size_t)k * LD + r];
-        T nr = fma(-lr, yr, br[q]);
-        nr = fma(li, yi, nr);
-        T ni = fma(-lr, yi, bi[q]);
-        ni = fma(-li, yr, ni);
-        const bool act = go && r > k && r < N;
-        br[q] = act ? nr : br[q];
-        bi[q] = act ? ni : bi[q];
+      for (int q = 0; q < R; ++q)
+#pragma unroll
+        for (int i = 0; i < B; ++i) {
+          lr[q][i] = nr_[q][i];
+          li[q][i] = ni_[q][i];
+        }
+      if (k0 > 0) {
+        columns<B>(Er, k0 - B, nr_);
+        columns<B>(Ei, k0 - B, ni_);
       }
-    }
-#pragma unroll 8
-    for (int k = N - 1; k >= 0; --k) {
-      const T vr = row_value(br, k), vi = row_value(bi, k);
-      const bool go = vr != T(0) || vi != T(0);
-      const T dr = Er[(size_t)k * LD + k], di = Ei[(size_t)k * LD + k];
-      // Smith's division (vr + i vi) / (dr + i di), as zgetrs divides
-      T xr, xi;
-      cdiv_t(vr, vi, dr, di, xr, xi);
 #pragma unroll
-      for (int q = 0; q < R; ++q) {
-        const int r = ln + 64 * q;
-        const T ur = Er[(size_t)k * LD + r], ui = Ei[(size_t)k * LD + r];
-        T nr = fma(-ur, xr, br[q]);
-        nr = fma(ui, xi, nr);
-        T ni = fma(-ur, xi, bi[q]);
-        ni = fma(-ui, xr, ni);
-        br[q] = go ? (r < k ? nr : (r == k ? xr : br[q])) : br[q];
-        bi[q] = go ? (r < k ? ni : (r == k ? xi : bi[q])) : bi[q];
+      for (int i = B - 1; i >= 0; --i) {
+        const int k = k0 + i;
+        T cr[R], ci[R];
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+          cr[q] = lr[q][i];
+          ci[q] = li[q][i];
+        }
+        const T vr = row_value(br, k), vi = row_value(bi, k);
+        const bool go = vr != T(0) || vi != T(0);
+        // Smith's division (vr + i vi) / (dr + i di), as zgetrs divides
+        T xr, xi;
+        cdiv_t(vr, vi, row_value(cr, k), row_value(ci, k), xr, xi);
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+          const int r = ln + 64 * q;
+          T nr = fma(-cr[q], xr, br[q]);
+          nr = fma(ci[q], xi, nr);
+          T ni = fma(-cr[q], xi, bi[q]);
+          ni = fma(-ci[q], xr, ni);
+          br[q] = go ? (r < k ? nr : (r == k ? xr : br[q])) : br[q];
+          bi[q] = go ? (r < k ? ni : (r == k ? xi : bi[q])) : bi[q];
+        }
       }
     }
   }

@@ -1429,15 +1429,15 @@ struct Radau {
   __device__ __forceinline__ MT* wE1() const { return ws; }
   __device__ __forceinline__ MT* wE2r() const { return ws + MLU::kMat; }
   __device__ __forceinline__ MT* wE2i() const { return ws + 2 * MLU::kMat; }
-  __device__ __forceinline__ int* wipiv1() const { return reinterpret_cast<int*>(ws + 3 * MLU::kMat); }
-  __device__ __forceinline__ int* wipiv2() const { return wipiv1() + N; }
+  __device__ __forceinline__ int* wperm1() const { return MLU::perm1(ws); }
+  __device__ __forceinline__ int* wperm2() const { return MLU::perm2(ws); }
 
   __device__ __forceinline__ void solve1(double (&b)[R]) const {
     if constexpr (kMemLU) {
       MT bb[R];
 #pragma unroll
       for (int q = 0; q < R; ++q) bb[q] = kMixed ? (MT)ldexp(b[q], -ex1[q]) : (MT)b[q];
-      MLU::solve_real(wE1(), wipiv1(), bb);
+      MLU::solve_real(wE1(), wperm1(), bb);
 #pragma unroll
       for (int q = 0; q < R; ++q) b[q] = kMixed ? ldexp((double)bb[q], -cx1[q]) : (double)bb[q];
     } else if constexpr (kRow16) {
@@ -1463,7 +1463,7 @@ struct Radau {
         xr[q] = kMixed ? (MT)ldexp(br[q], -ex2[q]) : (MT)br[q];
         xi[q] = kMixed ? (MT)ldexp(bi[q], -ex2[q]) : (MT)bi[q];
       }
-      MLU::solve_cplx(wE2r(), wE2i(), wipiv2(), xr, xi);
+      MLU::solve_cplx(wE2r(), wE2i(), wperm2(), xr, xi);
 #pragma unroll
       for (int q = 0; q < R; ++q) {
         br[q] = kMixed ? ldexp((double)xr[q], -cx2[q]) : (double)xr[q];
@@ -1722,7 +1722,7 @@ struct Radau {
         MT* w1 = wE1() + r;
         MT* w2r = wE2r() + r;
         MT* w2i = wE2i() + r;
-#pragma unroll 4
+#pragma unroll 16
         for (int j = 0; j < N; ++j) {
           // the column exponents are read across lanes (readlane), so with
           // every lane active: inside a branch on the row's validity the
@@ -1753,8 +1753,8 @@ struct Radau {
     }
     if constexpr (kMemLU) {
       wave_vmem_sync();  // every lane's rows before the panels read them
-      MLU::factor_real(wE1(), wipiv1(), info);
-      MLU::factor_cplx(wE2r(), wE2i(), wipiv2(), info2);
+      MLU::factor_real(wE1(), wperm1(), MLU::tmp(ws), info);
+      MLU::factor_cplx(wE2r(), wE2i(), wperm2(), MLU::tmp(ws), info2);
     } else if constexpr (kRow16) {
       row16_lu_real<N, MT>(E1[0], src1, rd1[0], info);
       row16_lu_cplx<N, MT>(E2r[0], E2i[0], src2, rd2r[0], rd2i[0], info2);

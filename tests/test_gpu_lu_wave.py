@@ -1,6 +1,6 @@
 """Pivot search of the one-wavefront LU (order 54) and of the 16-lane groups' LU
-(order 14, four matrices a wavefront) on candidates that agree in their leading
-32 bits: the search compares those first and the rest only among
+(order 14, four matrices a wavefront) and of the panels of the blocked LU (order
+112, two rows a lane) on candidates that agree in their leading 32 bits: the search compares those first and the rest only among
 the rows that attain the maximum.  Interchanges must be the oracle's dgetrf /
 zgetrf ones: the largest magnitude wins whichever bits decide it, and equal
 magnitudes go to the first row in LAPACK's current order.
@@ -12,7 +12,8 @@ import accelerint_amd as acc
 
 pytestmark = pytest.mark.gpu
 
-STEPS = [(54, 0), (54, 1), (54, 17), (54, 52), (14, 0), (14, 1), (14, 5), (14, 12)]
+STEPS = [(54, 0), (54, 1), (54, 17), (54, 52), (14, 0), (14, 1), (14, 5), (14, 12),
+         (112, 0), (112, 15), (112, 16), (112, 47), (112, 64), (112, 110)]
 
 
 @pytest.fixture
