@@ -50,7 +50,16 @@ __global__ __launch_bounds__(64) void k_factor_test(int num, const double* __res
   for (int i = 0; i < (N + 3) / 4; ++i) perm.w[i] = 0;
   T rdr[R], rdi[R];
   int info = 0;
-  if constexpr (CPLX) lu_cplx<N, G, R, T>(ar, ai, pos, perm, rdr, rdi, info);
+  if constexpr (G == 64 && R == 1) {
+    // the other factorization of the pair works on the same real parts
+    T br[R][N], bi[R][N], d[R], di[R];
+    int p2[R], inf2;
+    Perm<N> q;
+#pragma unroll
+    for (int j = 0; j < N; ++j) br[0][j] = ar[0][j], bi[0][j] = ai[0][j];
+    if constexpr (CPLX) wave_lu<N, T>(br, p2, q, d, inf2, ar, ai, pos, perm, rdr, rdi, info);
+    else wave_lu<N, T>(ar, pos, perm, rdr, info, br, bi, p2, q, d, di, inf2);
+  } else if constexpr (CPLX) lu_cplx<N, G, R, T>(ar, ai, pos, perm, rdr, rdi, info);
   else lu_real<N, G, R, T>(ar, pos, perm, rdr, info);
 #pragma unroll
   for (int q = 0; q < R; ++q) {

@@ -93,7 +93,7 @@ struct MemLU {
   }
 
   // Pivot of step c among the rows with position >= c: the row, wave-uniform.
-  // The leading 32 bits of the magnitudes decide (see wave_pivot); if no
+  // The leading 32 bits of the magnitudes decide (see wave_pivot2); if no
   // candidate compares (a NaN column) the row at position c stays, as idamax
   // returns its first index when nothing compares greater.
   __device__ __forceinline__ static int pivot(const T (&v)[R], const int (&pos)[R], int c) {

@@ -392,7 +392,7 @@ __device__ __forceinline__ void group_argmax(T& bv, int& bkey) {
 }
 
 
-// Pivot search of the register LU at G = 64, one row per lane (row = lane):
+// Pivot search of the register LU at G = 64, one row per lane (wave_pivot2, row = lane):
 // the first maximum of the magnitudes v over the active lanes in LAPACK's row
 // order (pos), as a wave-uniform lane, or -1 if no active lane holds a
 // comparable value (every candidate NaN).  The magnitudes are compared as
@@ -409,39 +409,54 @@ template <int CTRL>
 __device__ __forceinline__ unsigned dpp_max_u(unsigned v) {
   return max_u(v, (unsigned)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xf, 0xf, false));
 }
+// The lane among cand, the lanes whose keys equal the maximum m: decided by the
+// full magnitudes, then by the row order.
 template <class T>
-__device__ __forceinline__ int wave_pivot(T v, int pos, bool act) {
-  const unsigned key = act && v == v ? mag_hi(v) + 1u : 0u;  // 0: no candidate
-  unsigned m = dpp_max_u<kDppXor1>(key);
-  m = dpp_max_u<kDppXor2>(m);
-  m = dpp_max_u<kDppHalfMirror>(m);
-  m = dpp_max_u<kDppMirror>(m);
-  int x = (int)m, y = (int)m;
-  swap_row_pairs(x, y);
-  x = y = (int)max_u((unsigned)x, (unsigned)y);
-  swap_halves(x, y);
-  m = (unsigned)__builtin_amdgcn_readfirstlane((int)max_u((unsigned)x, (unsigned)y));
-  unsigned long long cand = __builtin_amdgcn_ballot_w64(key == m);
-  int lane = (int)__builtin_ctzll(cand);  // (the lane that holds the maximum: never empty)
-  if (__builtin_expect((cand & (cand - 1)) != 0, 0)) {
-    if (m == 0) return -1;
-    lane = -1;
-    T bv = T(0);
-    int best = 0;
-    while (cand) {
-      const int l = (int)__builtin_ctzll(cand);
-      cand &= cand - 1;
-      const T w = Grp<64>::bcast(v, l);
-      const int q = __builtin_amdgcn_readlane(pos, l);
-      if (lane < 0 || w > bv || (w == bv && q < best)) {
-        bv = w;
-        best = q;
-        lane = l;
-      }
+__device__ __forceinline__ int wave_pivot_tie(T v, int pos, unsigned m, unsigned long long cand) {
+  if (m == 0) return -1;
+  int lane = -1;
+  T bv = T(0);
+  int best = 0;
+  while (cand) {
+    const int l = (int)__builtin_ctzll(cand);
+    cand &= cand - 1;
+    const T w = Grp<64>::bcast(v, l);
+    const int q = __builtin_amdgcn_readlane(pos, l);
+    if (lane < 0 || w > bv || (w == bv && q < best)) {
+      bv = w;
+      best = q;
+      lane = l;
     }
-    lane = __builtin_amdgcn_readfirstlane(lane);
   }
-  return lane;
+  return __builtin_amdgcn_readfirstlane(lane);
+}
+// Two searches side by side: each is one chain of dependent lane exchanges.
+template <class T>
+__device__ __forceinline__ void wave_pivot2(T v, int pos, bool act, T v2, int pos2, bool act2, int& lane, int& lane2) {
+  const unsigned key = act && v == v ? mag_hi(v) + 1u : 0u;  // 0: no candidate
+  const unsigned key2 = act2 && v2 == v2 ? mag_hi(v2) + 1u : 0u;
+  unsigned m = dpp_max_u<kDppXor1>(key), m2 = dpp_max_u<kDppXor1>(key2);
+  m = dpp_max_u<kDppXor2>(m), m2 = dpp_max_u<kDppXor2>(m2);
+  m = dpp_max_u<kDppHalfMirror>(m), m2 = dpp_max_u<kDppHalfMirror>(m2);
+  m = dpp_max_u<kDppMirror>(m), m2 = dpp_max_u<kDppMirror>(m2);
+  int x = (int)m, y = (int)m, x2 = (int)m2, y2 = (int)m2;
+  swap_row_pairs(x, y);
+  swap_row_pairs(x2, y2);
+  x = y = (int)max_u((unsigned)x, (unsigned)y);
+  x2 = y2 = (int)max_u((unsigned)x2, (unsigned)y2);
+  swap_halves(x, y);
+  swap_halves(x2, y2);
+  m = (unsigned)__builtin_amdgcn_readfirstlane((int)max_u((unsigned)x, (unsigned)y));
+  m2 = (unsigned)__builtin_amdgcn_readfirstlane((int)max_u((unsigned)x2, (unsigned)y2));
+  const unsigned long long cand = __builtin_amdgcn_ballot_w64(key == m);
+  const unsigned long long cand2 = __builtin_amdgcn_ballot_w64(key2 == m2);
+  lane = (int)__builtin_ctzll(cand);  // (the lane that holds the maximum: never empty)
+  lane2 = (int)__builtin_ctzll(cand2);
+  const unsigned long long tie = cand & (cand - 1), tie2 = cand2 & (cand2 - 1);
+  if (__builtin_expect((tie | tie2) != 0, 0)) {
+    if (tie) lane = wave_pivot_tie(v, pos, m, cand);
+    if (tie2) lane2 = wave_pivot_tie(v2, pos2, m2, cand2);
+  }
 }
 
 // Tests of a wave-uniform pivot on its bits, in scalar registers.
@@ -466,7 +481,7 @@ __device__ __forceinline__ void pin_s(T& v) {
   __asm__ volatile("" : "+s"(v));
 }
 // Columns whose pivot-row entries are in scalar registers at once (the
-// schedule of a step is cut after every such chunk): more of them at once
+// updates of one chunk are pinned before the next one's): more of them at once
 // overflow the 102 scalar registers, and every spilled broadcast costs two
 // lane moves.
 constexpr int kBcastChunk = 8;
@@ -567,51 +582,82 @@ __device__ __forceinline__ void lu_init(int (&pos)[R], T (&rd)[R], int& info) {
   info = 0;
 }
 
-// Elimination step k of the real LU, a wavefront per matrix and a row per lane
-// (k a compile-time constant after unrolling): the operations of lu_real_step
+// Elimination step k of the real and the complex LU together, a wavefront per
+// pair of matrices and a row of each per lane (k a compile-time constant after
+// unrolling): for each matrix the operations of lu_real_step and lu_cplx_step
 // below in the same order.  Bound by the issue of a lane move per broadcast
-// pivot-row word and the step's chain search -> reciprocal -> multiplier.  What
-// a step leaves behind (multipliers, reciprocal, positions, pivot row) is
-// pinned to the step and the trailing update is cut into chunks of columns:
-// left alone, the compiler delayed the selects and updates of each step past
-// the next one's branches, which kept up to 54 broadcasts alive in scalar
-// registers (spilled by two lane moves each) and gave every step scratch slots.
-// With the solves' SolveView, order 54, 32768 conditions of one global step:
-// FP64 265 -> 117 ms (scratch 2816 -> 784 B a lane, lane moves 17000 -> 11700),
-// FP32 factors on 65536 conditions 253 -> 186 ms (scratch 912 -> 0 B).
+// pivot-row word and the step's chain search -> reciprocal -> multiplier; the
+// two chains are independent and are issued side by side.  What a step leaves
+// behind (multipliers, reciprocals, positions, pivot rows, updated columns) is
+// pinned to the step, column after column: left alone, the compiler delayed the
+// selects and updates of each step past the next one's branches, which kept up
+// to 54 broadcasts alive in scalar registers (spilled by two lane moves each)
+// and gave every step scratch slots.  Order 54, cycles for the pair of
+// factorizations with one wavefront per SIMD, one matrix after the other ->
+// together: FP64 181600 -> 176100, FP32 119100 -> 107700; 65536 conditions of
+// one global step with FP32 factors 155.6 -> 149.9 ms, 32768 in FP64
+// 103.0 -> 102.1 ms.  (Filling each chain's waits with the other matrix's
+// column updates was slower, 117000 cycles in FP32: a broadcast used at once
+// waits longer than the chain does.)
 template <int N, class T>
-__device__ __forceinline__ void wave_lu_real_step(const int k, T (&a)[N], int& pos, Perm<N>& perm, T& rd, int& info) {
+__device__ __forceinline__ void wave_lu_step(const int k, T (&a)[N], int& pos, Perm<N>& perm, T& rd, int& info,
+                                             T (&ar)[N], T (&ai)[N], int& pos2, Perm<N>& perm2, T& rdr, T& rdi,
+                                             int& info2) {
   const int ln = Grp<64>::lane();
-  const int win = wave_pivot(fabs(a[k]), pos, pos >= k);
-  const int plane = win & 63;
-  const int prow = win >= 0 ? win : 0xff;
-  const int pp = __builtin_amdgcn_readlane(pos, plane);
-  const int ppos = win >= 0 ? pp : 0x7fffff;
-  perm.set(k, prow);
-  pin_s(perm.w[k >> 2]);
+  int win, win2;
+  wave_pivot2(fabs(a[k]), pos, pos >= k, fabs(ar[k]) + fabs(ai[k]), pos2, pos2 >= k, win, win2);
+  const int plane = win & 63, plane2 = win2 & 63;
+  const int prow = win >= 0 ? win : 0xff, prow2 = win2 >= 0 ? win2 : 0xff;
+  const int pp = __builtin_amdgcn_readlane(pos, plane), pp2 = __builtin_amdgcn_readlane(pos2, plane2);
   const T piv = Grp<64>::bcast(a[k], plane);
-  const bool nz = !is_zero(piv);
-  info = !nz && info == 0 ? k + 1 : info;
-  pin(info);
-  const bool is_piv = ln == prow;
-  pos = is_piv ? k : (pos == k ? ppos : pos);  // LAPACK swaps rows k and ppos
-  pin(pos);
+  const T pr_ = Grp<64>::bcast(ar[k], plane2);
+  const T pi_ = Grp<64>::bcast(ai[k], plane2);
   const T rp = recip(piv);
+  T rr, ri;
+  crecip(pr_, pi_, rr, ri);
+  const int ppos = win >= 0 ? pp : 0x7fffff, ppos2 = win2 >= 0 ? pp2 : 0x7fffff;
+  perm.set(k, prow);
+  perm2.set(k, prow2);
+  const bool nz = !is_zero(piv), nz2 = !(is_zero(pr_) && is_zero(pi_));
+  info = !nz && info == 0 ? k + 1 : info;
+  info2 = !nz2 && info2 == 0 ? k + 1 : info2;
+  const bool is_piv = ln == prow, is_piv2 = ln == prow2;
+  pos = is_piv ? k : (pos == k ? ppos : pos);  // LAPACK swaps rows k and ppos
+  pos2 = is_piv2 ? k : (pos2 == k ? ppos2 : pos2);
   T lq = a[k] * rp;
   // LAPACK divides instead of scaling by the reciprocal when |pivot| < sfmin
   // (FP64 path only; the FP32 factors need no such care)
   if constexpr (std::is_same<T, double>::value)
     if (__builtin_expect(is_subnormal_or_zero(piv), 0)) lq = a[k] / piv;
   rd = is_piv ? (nz ? rp : T(0)) : rd;
-  pin(rd);
-  const bool act = nz && pos > k;
+  rdr = is_piv2 ? (nz2 ? rr : T(0)) : rdr;
+  rdi = is_piv2 ? (nz2 ? ri : T(0)) : rdi;
+  const bool act = nz && pos > k, act2 = nz2 && pos2 > k;
   a[k] = act ? lq : a[k];
   T l = act ? -lq : T(-0.0);
+  const T xr = ar[k], xi = ai[k];
+  const T vr = xr * rr - xi * ri;
+  const T vi = xr * ri + xi * rr;
+  ar[k] = act2 ? vr : xr;
+  ai[k] = act2 ? vi : xi;
+  T lr = act2 ? vr : T(0), li = act2 ? vi : T(0);
+  pin_s(perm.w[k >> 2]);
+  pin_s(perm2.w[k >> 2]);
+  pin(info);
+  pin(info2);
+  pin(pos);
+  pin(pos2);
+  pin(rd);
+  pin(rdr);
+  pin(rdi);
   pin(a[k]);
   pin(l);
+  pin(ar[k]);
+  pin(ai[k]);
+  pin(lr);
+  pin(li);
 #pragma unroll
   for (int j0 = k + 1; j0 < N; j0 += kBcastChunk) {
-    __builtin_amdgcn_sched_barrier(0);
     T u[kBcastChunk];
 #pragma unroll
     for (int j = j0; j < j0 + kBcastChunk; ++j)
@@ -623,7 +669,24 @@ __device__ __forceinline__ void wave_lu_real_step(const int k, T (&a)[N], int& p
         pin(a[j]);
       }
   }
-  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int j0 = k + 1; j0 < N; j0 += kBcastChunk) {
+    T ur[kBcastChunk], ui[kBcastChunk];
+#pragma unroll
+    for (int j = j0; j < j0 + kBcastChunk; ++j)
+      if (j < N) {
+        ur[j - j0] = Grp<64>::bcast(ar[j], plane2);
+        ui[j - j0] = Grp<64>::bcast(ai[j], plane2);
+      }
+#pragma unroll
+    for (int j = j0; j < j0 + kBcastChunk; ++j)
+      if (j < N) {
+        ar[j] = fma(li, ui[j - j0], fma(-lr, ur[j - j0], ar[j]));
+        ai[j] = fma(-li, ur[j - j0], fma(-lr, ui[j - j0], ai[j]));
+        pin(ar[j]);
+        pin(ai[j]);
+      }
+  }
 }
 
 template <int N, int G, int R, class T>
@@ -688,79 +751,11 @@ template <int N, int G, int R, class T>
 __device__ __forceinline__ void lu_real(T (&a)[R][N], int (&pos)[R], Perm<N>& perm,
                                         T (&rd)[R], int& info) {
   lu_init<N, G, R, T>(pos, rd, info);
-  if constexpr (G == 64 && R == 1) {
-    Perm<N> pm = {};  // built in scalar registers
-    int inf = 0;
 #pragma unroll
-    for (int k = 0; k < N; ++k) wave_lu_real_step<N, T>(k, a[0], pos[0], pm, rd[0], inf);
-    perm = pm;
-    info = inf;
-  } else {
-#pragma unroll
-    for (int k = 0; k < N; ++k) lu_real_step<N, G, R, T>(k, a, pos, perm, rd, info);
-  }
+  for (int k = 0; k < N; ++k) lu_real_step<N, G, R, T>(k, a, pos, perm, rd, info);
 }
 
 // ---- complex LU (zgetf2 semantics) -------------------------------------------
-// (a wavefront per matrix, a row per lane: as wave_lu_real_step)
-template <int N, class T>
-__device__ __forceinline__ void wave_lu_cplx_step(const int k, T (&ar)[N], T (&ai)[N], int& pos, Perm<N>& perm, T& rdr,
-                                                  T& rdi, int& info) {
-  const int ln = Grp<64>::lane();
-  const int win = wave_pivot(fabs(ar[k]) + fabs(ai[k]), pos, pos >= k);
-  const int plane = win & 63;
-  const int prow = win >= 0 ? win : 0xff;
-  const int pp = __builtin_amdgcn_readlane(pos, plane);
-  const int ppos = win >= 0 ? pp : 0x7fffff;
-  perm.set(k, prow);
-  pin_s(perm.w[k >> 2]);
-  const T pr_ = Grp<64>::bcast(ar[k], plane);
-  const T pi_ = Grp<64>::bcast(ai[k], plane);
-  const bool nz = !(is_zero(pr_) && is_zero(pi_));
-  info = !nz && info == 0 ? k + 1 : info;
-  pin(info);
-  const bool is_piv = ln == prow;
-  pos = is_piv ? k : (pos == k ? ppos : pos);
-  pin(pos);
-  T rr, ri;
-  crecip(pr_, pi_, rr, ri);
-  rdr = is_piv ? (nz ? rr : T(0)) : rdr;
-  rdi = is_piv ? (nz ? ri : T(0)) : rdi;
-  pin(rdr);
-  pin(rdi);
-  const bool act = nz && pos > k;
-  const T xr = ar[k], xi = ai[k];
-  const T vr = xr * rr - xi * ri;
-  const T vi = xr * ri + xi * rr;
-  ar[k] = act ? vr : xr;
-  ai[k] = act ? vi : xi;
-  T lr = act ? vr : T(0), li = act ? vi : T(0);
-  pin(ar[k]);
-  pin(ai[k]);
-  pin(lr);
-  pin(li);
-#pragma unroll
-  for (int j0 = k + 1; j0 < N; j0 += kBcastChunk) {
-    __builtin_amdgcn_sched_barrier(0);
-    T ur[kBcastChunk], ui[kBcastChunk];
-#pragma unroll
-    for (int j = j0; j < j0 + kBcastChunk; ++j)
-      if (j < N) {
-        ur[j - j0] = Grp<64>::bcast(ar[j], plane);
-        ui[j - j0] = Grp<64>::bcast(ai[j], plane);
-      }
-#pragma unroll
-    for (int j = j0; j < j0 + kBcastChunk; ++j)
-      if (j < N) {
-        ar[j] = fma(li, ui[j - j0], fma(-lr, ur[j - j0], ar[j]));
-        ai[j] = fma(-li, ur[j - j0], fma(-lr, ui[j - j0], ai[j]));
-        pin(ar[j]);
-        pin(ai[j]);
-      }
-  }
-  __builtin_amdgcn_sched_barrier(0);
-}
-
 template <int N, int G, int R, class T>
 __device__ __forceinline__ void lu_cplx_step(const int k, T (&ar)[R][N], T (&ai)[R][N], int (&pos)[R],
                                              Perm<N>& perm, T (&rdr)[R], T (&rdi)[R], int& info) {
@@ -837,17 +832,28 @@ __device__ __forceinline__ void lu_cplx(T (&ar)[R][N], T (&ai)[R][N], int (&pos)
   lu_init<N, G, R, T>(pos, rdr, info);
 #pragma unroll
   for (int q = 0; q < R; ++q) rdi[q] = T(0);
-  if constexpr (G == 64 && R == 1) {
-    Perm<N> pm = {};
-    int inf = 0;
 #pragma unroll
-    for (int k = 0; k < N; ++k) wave_lu_cplx_step<N, T>(k, ar[0], ai[0], pos[0], pm, rdr[0], rdi[0], inf);
-    perm = pm;
-    info = inf;
-  } else {
+  for (int k = 0; k < N; ++k) lu_cplx_step<N, G, R, T>(k, ar, ai, pos, perm, rdr, rdi, info);
+}
+
+// The real and the complex LU of a 64-lane group, a row per lane, step by step
+// together.
+template <int N, class T>
+__device__ __forceinline__ void wave_lu(T (&a)[1][N], int (&pos)[1], Perm<N>& perm, T (&rd)[1], int& info,
+                                        T (&ar)[1][N], T (&ai)[1][N], int (&pos2)[1], Perm<N>& perm2, T (&rdr)[1],
+                                        T (&rdi)[1], int& info2) {
+  lu_init<N, 64, 1, T>(pos, rd, info);
+  lu_init<N, 64, 1, T>(pos2, rdr, info2);
+  rdi[0] = T(0);
+  Perm<N> pm = {}, pm2 = {};  // built in scalar registers
+  int inf = 0, inf2 = 0;
 #pragma unroll
-    for (int k = 0; k < N; ++k) lu_cplx_step<N, G, R, T>(k, ar, ai, pos, perm, rdr, rdi, info);
-  }
+  for (int k = 0; k < N; ++k)
+    wave_lu_step<N, T>(k, a[0], pos[0], pm, rd[0], inf, ar[0], ai[0], pos2[0], pm2, rdr[0], rdi[0], inf2);
+  perm = pm;
+  perm2 = pm2;
+  info = inf;
+  info2 = inf2;
 }
 
 // ---- triangular solves (dgetrs / zgetrs, nrhs = 1) ---------------------------
@@ -1758,9 +1764,9 @@ struct Radau {
     } else if constexpr (kRow16) {
       row16_lu_real<N, MT>(E1[0], src1, rd1[0], info);
       row16_lu_cplx<N, MT>(E2r[0], E2i[0], src2, rd2r[0], rd2i[0], info2);
+    } else if constexpr (G == 64 && R == 1) {
+      wave_lu<N, MT>(E1, pos1, perm1, rd1, info, E2r, E2i, pos2, perm2, rd2r, rd2i, info2);
     } else {
-      // (interleaving the two factorizations' steps was measured slower at
-      // N = 54: the larger live set spills)
       lu_real<N, G, R, MT>(E1, pos1, perm1, rd1, info);
       lu_cplx<N, G, R, MT>(E2r, E2i, pos2, perm2, rd2r, rd2i, info2);
     }
