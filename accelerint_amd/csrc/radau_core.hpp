@@ -594,9 +594,11 @@ __device__ __forceinline__ void lu_init(int (&pos)[R], T (&rd)[R], int& info) {
 // to 54 broadcasts alive in scalar registers (spilled by two lane moves each)
 // and gave every step scratch slots.  Order 54, cycles for the pair of
 // factorizations with one wavefront per SIMD, one matrix after the other ->
-// together: FP64 181600 -> 176100, FP32 119100 -> 107700; 65536 conditions of
-// one global step with FP32 factors 155.6 -> 149.9 ms, 32768 in FP64
-// 103.0 -> 102.1 ms.  (Filling each chain's waits with the other matrix's
+// together: FP64 181600 -> 178700, FP32 119100 -> 107700; 65536 conditions of
+// one global step with FP32 factors 155.6 -> 149.1 ms, 32768 in FP64
+// 103.0 -> 102.6 ms.  (In FP64 the schedule is cut around the updates: without
+// the cuts 176100 cycles, but the longer live ranges cost the kernel that holds
+// all three networks 1%.  Filling each chain's waits with the other matrix's
 // column updates was slower, 117000 cycles in FP32: a broadcast used at once
 // waits longer than the chain does.)
 template <int N, class T>
@@ -656,6 +658,7 @@ __device__ __forceinline__ void wave_lu_step(const int k, T (&a)[N], int& pos, P
   pin(ai[k]);
   pin(lr);
   pin(li);
+  if constexpr (std::is_same<T, double>::value) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
   for (int j0 = k + 1; j0 < N; j0 += kBcastChunk) {
     T u[kBcastChunk];
@@ -687,6 +690,7 @@ __device__ __forceinline__ void wave_lu_step(const int k, T (&a)[N], int& pos, P
         pin(ai[j]);
       }
   }
+  if constexpr (std::is_same<T, double>::value) __builtin_amdgcn_sched_barrier(0);
 }
 
 template <int N, int G, int R, class T>
