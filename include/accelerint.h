@@ -275,10 +275,12 @@ int accelerInt_eval_callbacks(int NUM, double t, const double *y_host, const dou
                               double *dy_host, double *jac_host);
 
 /* Test hook, no counterpart in the reference's API: factors NUM matrices of
- * order n (2, 14 or 54) on the device with the LU the integrator runs at that
- * order and precision (a row per lane with implicit interchanges, LAPACK's
- * pivot rule; at order 54 the real and the complex LU step by step together,
- * the other one on the same matrix) and returns them in the form of LAPACK dgetrf_ / zgetrf_, the calls of RK_Decomp (radau2a.c:273,277):
+ * order n (2, 14, 54 or 112) on the device with the LU the integrator runs at
+ * that order and precision (implicit interchanges with LAPACK's pivot rule: a
+ * row per lane up to order 54, the workspace LU at 112; at order 54 the real
+ * and the complex LU step by step together, the other one on the same matrix)
+ * and returns them in the form of LAPACK dgetrf_ / zgetrf_, the calls of
+ * RK_Decomp (radau2a.c:273,277):
  * a_re / a_im are NUM row-major n x n matrices (a_im NULL: real LU; else the
  * imaginary parts of a complex LU); lu_re / lu_im receive the combined unit-L
  * / U factors of P A, row-major; ipiv[c*n + k] the 1-based row interchanged
